@@ -30,6 +30,7 @@
 
 #include "common.hpp"
 #include "gf2x.hpp"
+#include "jump_blocks.hpp"
 #include "kernels.hpp"
 #include "runtime.hpp"
 
@@ -547,26 +548,6 @@ std::vector<uint16_t> jump_mask16(const std::vector<uint32_t> &w) {
     return m;
 }
 
-std::vector<uint32_t> words_from_mask16(const std::vector<uint16_t> &m, int nwords) {
-    std::vector<uint32_t> w((size_t)nwords, 0);
-    const size_t nchunks = m.size() / 64;
-    for (size_t c = 0; c < nchunks; c++) {
-        uint64_t rows[16] = {};
-        const uint16_t *mc = m.data() + c * 64;
-        for (int rho = 0; rho < 64; rho++)
-            for (int q = 0; q < 16; q++)
-                rows[q] |= (uint64_t)((mc[rho] >> q) & 1u) << rho;
-        for (int q = 0; q < 16; q++) {
-            const size_t i = c * 32 + 2 * (size_t)q;
-            if (i < w.size())
-                w[i] = (uint32_t)rows[q];
-            if (i + 1 < w.size())
-                w[i + 1] = (uint32_t)(rows[q] >> 32);
-        }
-    }
-    return w;
-}
-
 int append_jump_masks16(const std::vector<const std::vector<uint16_t> *> &ms, std::vector<uint64_t> &out) {
     size_t n = 64;
     for (const auto *m : ms)
@@ -633,7 +614,6 @@ JumpCache::JumpCache(Context &c, const std::vector<int> &slots, uint64_t cell, i
         e.mod = modulus_for(c, keys[(size_t)i]);
         e.words32 = (int)((e.mod->deg() + 31) / 32);
         e.pow2.push_back(e.mod->xpow(cell));
-        e.t1.resize(B_);
         e.t1w.resize(B_);
         if (!far)
             return;
@@ -654,7 +634,6 @@ JumpCache::JumpCache(Context &c, const std::vector<int> &slots, uint64_t cell, i
             if (k > 0) {
                 cur = k == k0 ? cur : e.mod->mulmod(cur, e.pow2[0]);
                 e.t1w[k] = gf2::to_words32(cur, e.words32);
-                e.t1[k] = jump_mask16(e.t1w[k]);
             }
         }
     });
@@ -685,7 +664,7 @@ std::shared_ptr<JumpCache> JumpCache::shared(Context &c, const std::vector<int> 
     return p;
 }
 
-bool JumpCache::get_masks(int slot, uint64_t pos, std::vector<uint16_t> &m16, bool cheap) const {
+bool JumpCache::get(int slot, uint64_t pos, std::vector<uint32_t> &words, bool cheap) const {
     if (pos == 0 || pos % cell_)
         return false;
     auto it = entries_.find(slot);
@@ -694,7 +673,7 @@ bool JumpCache::get_masks(int slot, uint64_t pos, std::vector<uint16_t> &m16, bo
     const Entry &e = it->second;
     const uint64_t k = pos / cell_;
     if (k < B_) {
-        m16 = e.t1[(size_t)k];
+        words = e.t1w[(size_t)k];
         return true;
     }
     if (cheap)
@@ -702,8 +681,7 @@ bool JumpCache::get_masks(int slot, uint64_t pos, std::vector<uint16_t> &m16, bo
     const uint64_t j = k / B_, r = k % B_;
     gf2::Poly acc;
     if (j < e.t2p.size()) {
-        acc = r ? e.mod->mulmod(e.t2p[(size_t)j], poly_of_words32(words_from_mask16(e.t1[(size_t)r], e.words32)))
-                : e.t2p[(size_t)j];
+        acc = r ? e.mod->mulmod(e.t2p[(size_t)j], poly_of_words32(e.t1w[(size_t)r])) : e.t2p[(size_t)j];
     } else {
         if (k >> e.pow2.size())
             return false;
@@ -711,7 +689,15 @@ bool JumpCache::get_masks(int slot, uint64_t pos, std::vector<uint16_t> &m16, bo
             if (k >> i & 1)
                 acc = acc.empty() ? e.pow2[i] : e.mod->mulmod(acc, e.pow2[i]);
     }
-    m16 = jump_mask16(gf2::to_words32(acc, e.words32));
+    words = gf2::to_words32(acc, e.words32);
+    return true;
+}
+
+bool JumpCache::get_masks(int slot, uint64_t pos, std::vector<uint16_t> &m16, bool cheap) const {
+    std::vector<uint32_t> words;
+    if (!get(slot, pos, words, cheap))
+        return false;
+    m16 = jump_mask16(words);
     return true;
 }
 
@@ -722,15 +708,6 @@ const std::vector<uint32_t> *JumpCache::table_words(int slot, uint64_t pos) cons
     if (it == entries_.end() || pos / cell_ >= B_)
         return nullptr;
     return &it->second.t1w[(size_t)(pos / cell_)];
-}
-
-bool JumpCache::get(int slot, uint64_t pos, std::vector<uint32_t> &words, bool cheap) const {
-    std::vector<uint16_t> m16;
-    if (!get_masks(slot, pos, m16, cheap))
-        return false;
-    auto it = entries_.find(slot);
-    words = words_from_mask16(m16, it->second.words32);
-    return true;
 }
 
 namespace {
@@ -771,6 +748,54 @@ constexpr int kAutoCacheCells = 64;
 constexpr int kAutoCacheMaxK = 2048;
 // Cells per block of an incremental polynomial chain on the host pool.
 constexpr size_t kChainMin = 32;
+
+// Partial windows of one round of blocked jumps, at most: they stay in the
+// 256 MB last-level cache between the products and the folds, and a plan of
+// any number of jumps needs no more memory for them.
+constexpr size_t kPartBytes = (size_t)128 << 20;
+
+// The tiles of one launch's groups [g0, g1) and the workgroups' shares of
+// them: kTilesPerCu workgroups per CU (the kernel's occupancy) with about the
+// same number of products each, so that one round of workgroups does the
+// launch and each makes its base's planes about once.  A tile of up to 32
+// columns does half the products of a wider one.
+constexpr int kTilesPerCu = 2;
+static void jb_tiles(const std::vector<JumpBlocks> &groups, int g0, int g1, int bits, int cus,
+                     std::vector<JumpTile> &tiles, std::vector<JumpShare> &shares) {
+    const int first = (int)tiles.size();
+    int64_t total = 0;
+    auto weight = [&](const JumpTile &t) { return groups[(size_t)t.group].ncols - t.c0 > 32 ? 2 : 1; };
+    for (int g = g0; g < g1; g++)
+        for (int plane = 0; plane < bits / 32; plane++)
+            for (int c0 = 0; c0 < groups[(size_t)g].ncols; c0 += kJbCols) {
+                tiles.push_back(JumpTile{g, c0, groups[(size_t)g].param, plane});
+                total += weight(tiles.back()) * (jb_plane_words(groups[(size_t)g].n) / kJbGroup);
+            }
+    const int64_t count = std::max<int64_t>(1, std::min<int64_t>(total, (int64_t)kTilesPerCu * cus));
+    JumpShare S{-1, 0, 0, 0, {}};
+    int64_t done = 0, made = 0;
+    for (int t = first; t < (int)tiles.size(); t++) {
+        const int w = weight(tiles[(size_t)t]), n = jb_plane_words(groups[(size_t)tiles[(size_t)t].group].n) / kJbGroup;
+        for (int at = 0; at < n;) {
+            if (S.tile0 < 0)
+                S.tile0 = t, S.g0 = at, S.first = tiles[(size_t)t];
+            // up to the end of the share: total * (made + 1) / count
+            const int64_t end = total * (made + 1) / count;
+            const int take = (int)std::min<int64_t>(n - at, std::max<int64_t>(1, (end - done + w - 1) / w));
+            at += take;
+            done += (int64_t)take * w;
+            S.tile1 = t, S.g1 = at;
+            if (done >= end) {
+                shares.push_back(S);
+                S.tile0 = -1;
+                while (made + 1 < count && done >= total * (made + 1) / count)
+                    made++;
+            }
+        }
+    }
+    if (S.tile0 >= 0)
+        shares.push_back(S);
+}
 
 GridModel grid_model_of(int bits, int cls, int mexp, int n) {
     GridModel m;
@@ -1074,12 +1099,34 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
             cache = auto_cache.get();
         }
     }
+    // Batched jumps of a generator: in coefficient blocks on the matrix cores
+    // (at least jump_mfma_min of them), or by the word-XOR kernel, which takes
+    // the coefficients as per-residue masks.
+    std::vector<char> blocked((size_t)G, 0);
+    for (int g = 0; g < G && masks && c.jump_mfma_min > 0; g++) {
+        int need = 0;
+        for (const Cell &cl : cells[(size_t)g])
+            need += cl.start > 0;
+        blocked[(size_t)g] = need >= c.jump_mfma_min;
+    }
+    // (blocked jumps read table entries in place)
     auto cached = [&](int g, size_t k, bool cheap) {
         const int slot = gens[(size_t)g].slot;
         const uint64_t pos = cells[(size_t)g][k].start;
-        return masks ? cache->get_masks(slot, pos, m16[(size_t)g][k], cheap)
-                     : cache->get(slot, pos, polys[(size_t)g][k], cheap);
+        if (masks && !blocked[(size_t)g])
+            return cache->get_masks(slot, pos, m16[(size_t)g][k], cheap);
+        if (masks && cache->table_words(slot, pos))
+            return true;
+        return cache->get(slot, pos, polys[(size_t)g][k], cheap);
     };
+    auto words_of = [&](int g, size_t k) {
+        const std::vector<uint32_t> *w = &polys[(size_t)g][k];
+        if (w->empty() && cache)
+            if (const auto *tw = cache->table_words(gens[(size_t)g].slot, cells[(size_t)g][k].start))
+                w = tw;
+        return w;
+    };
+    auto ready = [&](int g, size_t k) { return !words_of(g, k)->empty() || !m16[(size_t)g][k].empty(); };
     std::vector<int> compute;                      // generators with cells off the cache
     std::vector<std::pair<int, size_t>> composed;  // cells the cache makes with one product
     for (int g = 0; g < G; g++) {
@@ -1106,7 +1153,7 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
     // A cell the cache could not make (its set is not in the cache, or the
     // position is beyond it) is computed below with its generator's others.
     for (const auto &gk : composed)
-        if (polys[(size_t)gk.first][gk.second].empty() && m16[(size_t)gk.first][gk.second].empty() &&
+        if (!ready(gk.first, gk.second) &&
             std::find(compute.begin(), compute.end(), gk.first) == compute.end())
             compute.push_back(gk.first);
     // The rest incrementally along each generator (x^b = x^a * x^(b - a)),
@@ -1123,7 +1170,7 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
             const auto &cv = cells[(size_t)g];
             std::vector<size_t> ks;
             for (size_t k = 0; k < cv.size(); k++)
-                if (cv[k].start > 0 && polys[(size_t)g][k].empty() && m16[(size_t)g][k].empty())
+                if (cv[k].start > 0 && !ready(g, k))
                     ks.push_back(k);
             // blocks of at least kChainMin cells: a block's first power costs
             // about as much as that many products
@@ -1157,7 +1204,7 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
             }
             cur_off = off;
             out[k] = gf2::to_words32(cur, pw);
-            if (masks)
+            if (masks && !blocked[(size_t)g])
                 m16[(size_t)g][k] = jump_mask16(out[k]);
         }
     });
@@ -1169,26 +1216,24 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
         int nchunks;
     };
     std::vector<Group> groups;
-    // Matrix-core groups: all of a generator's jumps (both phases: the
-    // two-phase launch runs them with phase 0), one bit-plane pass each.
-    struct MGroup {
-        int g, phase;
+    // Blocked jumps: all of a generator's (both phases: the two-phase launch
+    // runs them with phase 0).
+    struct BGroup {
+        int g;
         std::vector<size_t> cells;
     };
-    std::vector<MGroup> mg;
+    std::vector<BGroup> bg;
     std::vector<uint64_t> mask_host;
     std::vector<uint32_t> poly_host;
     if (masks) {
         for (int g = 0; g < G; g++) {
-            if (gens[(size_t)g].bits == 32 && c.jump_mfma_min > 0) {
+            if (blocked[(size_t)g]) {
                 std::vector<size_t> need;
                 for (size_t k = 0; k < cells[(size_t)g].size(); k++)
                     if (cells[(size_t)g][k].start > 0)
                         need.push_back(k);
-                if ((int)need.size() >= c.jump_mfma_min) {
-                    mg.push_back(MGroup{g, 0, need});
-                    continue;
-                }
+                bg.push_back(BGroup{g, need});
+                continue;
             }
             for (int ph = 0; ph < 2; ph++) {
                 std::vector<size_t> need;
@@ -1258,93 +1303,97 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
         }
         arena_bytes += align256((size_t)P * nb * sbytes);
     }
-    // Matrix-core groups: planes and jumped windows in the arena, the
-    // coefficient words of every jump transposed ([word][jump]).
-    mgroups.clear();
-    mitems.clear();
-    mgroup_gen.clear();
-    for (auto &r : mrange)
-        r = MRange{};
-    mjumps = 0;
-    std::vector<uint32_t> coef_host;
+    // Blocked jumps: a generator's jumps as one JumpBlocks group, split where
+    // the partial windows of one round would outgrow kPartBytes.  Polynomials
+    // go up as they are, zero-padded to whole blocks; the jumped windows and
+    // (reused by every round) the partial windows lie in the arena.
+    bgroups.clear();
+    bgroup_gen.clear();
+    blaunches.clear();
+    mjumps = mgroups = 0;
+    std::vector<JumpTile> btiles;
+    std::vector<JumpShare> bshares;
+    std::vector<JumpFold> bfolds;
+    size_t bcoef_words = 0;
+    struct BCopy {
+        size_t at;
+        const std::vector<uint32_t> *w;
+    };
+    std::vector<BCopy> bcopies;
     {
-        std::stable_sort(mg.begin(), mg.end(), [](const MGroup &a, const MGroup &b) { return a.phase < b.phase; });
-        std::vector<MJumpItem> mit[kMjRowTiles + 1][2];
-        for (const MGroup &m : mg) {
+        std::stable_sort(bg.begin(), bg.end(), [&](const BGroup &a, const BGroup &b) {
+            return group_of(gens[(size_t)a.g]) < group_of(gens[(size_t)b.g]);
+        });
+        size_t round_bytes = 0, most = 0;
+        for (const BGroup &m : bg) {
             const GenRef &ref = gens[(size_t)m.g];
-            const int nj = (int)m.cells.size();
-            const int njp = (nj + 31) / 32 * 32;
-            const int kpad = mj_kpad(ref.mexp);
-            const int wc = kpad / 32, pw = mj_pw(kpad, ref.n);
-            const size_t sbytes = (size_t)ref.n * 4;
-            MJumpGroup gr{};
-            gr.state_in = (uint64_t)(uintptr_t)ref.state_in;
-            gr.in_parts = 1;
-            gr.planes = arena_bytes;  // fixed up below
-            arena_bytes += align256((size_t)pw * 32 * 4);
-            gr.out = arena_bytes;  // fixed up below
-            gr.out_stride = sbytes;
-            for (int b = 0; b < nj; b++)
-                slot_of[{m.g, m.cells[(size_t)b]}] = std::make_tuple((uint64_t)(arena_bytes + (size_t)b * sbytes), 1,
-                                                                     (uint64_t)0);
-            arena_bytes += align256((size_t)nj * sbytes);
-            gr.coef = (uint64_t)coef_host.size() * 4;  // fixed up below
-            coef_host.resize(coef_host.size() + (size_t)wc * (size_t)njp, 0u);
-            uint32_t *cf = coef_host.data() + gr.coef / 4;
-            // jump b's words in column b: the cell's own words, the cache's
-            // table entry, or converted from the mask form (on the host
-            // pool); then the array row by row
-            std::vector<const std::vector<uint32_t> *> wv((size_t)nj);
-            std::vector<std::vector<uint32_t>> conv((size_t)nj);
-            parallel_for(nj, [&](int b) {
-                const size_t k = m.cells[(size_t)b];
-                const std::vector<uint32_t> *w = &polys[(size_t)m.g][k];
-                if (w->empty() && cache)
-                    if (const auto *tw = cache->table_words(ref.slot, cells[(size_t)m.g][k].start))
-                        w = tw;
-                if (w->empty()) {
-                    conv[(size_t)b] = words_from_mask16(m16[(size_t)m.g][k], (ref.mexp + 31) / 32);
-                    w = &conv[(size_t)b];
-                }
-                wv[(size_t)b] = w;
-            });
-            parallel_for((wc + 15) / 16, [&](int blk) {
-                for (int x = 16 * blk; x < std::min(wc, 16 * blk + 16); x++) {
-                    uint32_t *row = cf + (size_t)x * (size_t)njp;
-                    for (int b = 0; b < nj; b++)
-                        row[b] = (size_t)x < wv[(size_t)b]->size() ? (*wv[(size_t)b])[(size_t)x] : 0u;
-                }
-            });
-            gr.nj = nj;
-            gr.njp = njp;
-            gr.kpad = kpad;
-            gr.pw = pw;
-            gr.param = ref.slot;
-            gr.n = ref.n;
-            const int gi = (int)mgroups.size();
-            mgroups.push_back(gr);
-            mgroup_gen.push_back(m.g);
-            for (int r0 = 0; r0 < nj; r0 += 32 * kMjRowTiles) {
-                const int rt = std::min(kMjRowTiles, (nj - r0 + 31) / 32);
-                for (int j0 = 0; j0 < ref.n; j0 += mj_words(rt))
-                    mit[rt][m.phase].push_back(MJumpItem{gi, r0, j0, 0});
+            if (ref.bits == 32) {
+                mgroups++;
+                mjumps += (int)m.cells.size();
             }
-            mjumps += nj;
+            const DevParam &D = c.param(ref.slot);
+            const int cls = c.class_of(ref.slot);
+            const int ch = jb_blocks(ref.mexp);
+            const size_t jbytes = (size_t)ch * (size_t)jb_part_words(ref.bits, ref.n) * 4;
+            const size_t sbytes = (size_t)ref.n * (size_t)(ref.bits / 8);
+            for (size_t b0 = 0; b0 < m.cells.size();) {
+                const size_t fit = round_bytes < kPartBytes ? (kPartBytes - round_bytes) / jbytes : 0;
+                const size_t nj = std::min(m.cells.size() - b0, std::max<size_t>(fit, round_bytes ? 0 : 1));
+                if (nj == 0) {
+                    round_bytes = 0;
+                    continue;
+                }
+                JumpBlocks gr{};
+                gr.state_in = (uint64_t)(uintptr_t)ref.state_in;
+                gr.coef = 4 * (uint64_t)bcoef_words;  // fixed up below
+                gr.parts = round_bytes;               // fixed up below
+                gr.out = arena_bytes;                 // fixed up below
+                gr.out_stride = sbytes;
+                gr.ncols = (int32_t)nj * ch;
+                gr.ch = ch;
+                gr.param = ref.slot;
+                gr.n = ref.n;
+                // a round's launches: one pair per (word size, class)
+                if (blaunches.empty() || round_bytes == 0 || blaunches.back().bits != ref.bits ||
+                    blaunches.back().cls != cls) {
+                    BLaunch L;
+                    L.bits = ref.bits;
+                    L.cls = cls;
+                    L.step = 1024;
+                    L.g0 = (int)bgroups.size();
+                    blaunches.push_back(L);
+                }
+                BLaunch &L = blaunches.back();
+                L.step = std::min(L.step, jb_step(ref.bits, cls, ref.n, D.pos));
+                L.f1 += (int)nj;
+                const int gi = (int)bgroups.size();
+                L.g1 = gi + 1;
+                for (size_t b = 0; b < nj; b++) {
+                    const size_t k = m.cells[b0 + b];
+                    slot_of[{m.g, k}] = std::make_tuple((uint64_t)(arena_bytes + b * sbytes), 1, (uint64_t)0);
+                    bcopies.push_back(BCopy{bcoef_words + b * (size_t)ch * kJbWords, words_of(m.g, k)});
+                    bfolds.push_back(JumpFold{gi, (int32_t)b});
+                }
+                bgroups.push_back(gr);
+                bgroup_gen.push_back(m.g);
+                bcoef_words += nj * (size_t)ch * kJbWords;
+                arena_bytes += align256(nj * sbytes);
+                round_bytes += align256(nj * jbytes);
+                most = std::max(most, round_bytes);
+                b0 += nj;
+            }
         }
-        int n0 = 0;
-        for (const MGroup &m : mg)
-            n0 += m.phase == 0;
-        mrange[0].g0 = 0, mrange[0].g1 = n0;
-        mrange[1].g0 = n0, mrange[1].g1 = (int)mg.size();
-        mrange[2].g0 = 0, mrange[2].g1 = (int)mg.size();
-        for (int rt = 1; rt <= kMjRowTiles; rt++) {
-            mrange[2].i0[rt] = (int)mitems.size();
-            for (int ph = 0; ph < 2; ph++) {
-                mrange[ph].i0[rt] = (int)mitems.size();
-                mitems.insert(mitems.end(), mit[rt][ph].begin(), mit[rt][ph].end());
-                mrange[ph].i1[rt] = (int)mitems.size();
-            }
-            mrange[2].i1[rt] = (int)mitems.size();
+        const uint64_t parts_at = arena_bytes;
+        arena_bytes += most;
+        int f = 0;
+        for (BLaunch &L : blaunches) {
+            L.f0 = f;
+            f = L.f1 += f;
+            for (int gi = L.g0; gi < L.g1; gi++)
+                bgroups[(size_t)gi].parts += parts_at;
+            L.s0 = (int)bshares.size();
+            jb_tiles(bgroups, L.g0, L.g1, L.bits, c.cus, btiles, bshares);
+            L.s1 = (int)bshares.size();
         }
     }
     // Items, one per cell.
@@ -1447,13 +1496,15 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
     const size_t o_polys = align256(o_segs + segs.size() * sizeof(Segment));
     const size_t o_masks = align256(o_polys + poly_host.size() * 4);
     const size_t o_jitems = align256(o_masks + mask_host.size() * 8);
-    const size_t o_mgroups = align256(o_jitems + jitems.size() * sizeof(JumpItem));
-    const size_t o_mitems = align256(o_mgroups + mgroups.size() * sizeof(MJumpGroup));
-    const size_t o_coef = align256(o_mitems + mitems.size() * sizeof(MJumpItem));
-    const size_t work_bytes = align256(o_coef + coef_host.size() * 4);
+    const size_t o_bgroups = align256(o_jitems + jitems.size() * sizeof(JumpItem));
+    const size_t o_btiles = align256(o_bgroups + bgroups.size() * sizeof(JumpBlocks));
+    const size_t o_bshares = align256(o_btiles + btiles.size() * sizeof(JumpTile));
+    const size_t o_bfolds = align256(o_bshares + bshares.size() * sizeof(JumpShare));
+    const size_t o_bcoef = align256(o_bfolds + bfolds.size() * sizeof(JumpFold));
+    const size_t work_bytes = align256(o_bcoef + bcoef_words * 4);
     this->o_items = o_items;
     this->o_jitems = o_jitems;
-    this->o_mgroups = o_mgroups;
+    this->o_bgroups = o_bgroups;
     wait_upload();
     grow_device(d_work, work_cap, work_bytes, "hipMalloc plan workspace");
     grow_pinned(h_stage, stage_cap, work_bytes);
@@ -1466,8 +1517,10 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
     const uint64_t dw = (uint64_t)(uintptr_t)d_work;
     d_items = reinterpret_cast<Item *>(d_work + o_items);
     d_jitems = reinterpret_cast<JumpItem *>(d_work + o_jitems);
-    d_mgroups = reinterpret_cast<MJumpGroup *>(d_work + o_mgroups);
-    d_mitems = reinterpret_cast<MJumpItem *>(d_work + o_mitems);
+    d_bgroups = reinterpret_cast<JumpBlocks *>(d_work + o_bgroups);
+    d_btiles = reinterpret_cast<JumpTile *>(d_work + o_btiles);
+    d_bshares = reinterpret_cast<JumpShare *>(d_work + o_bshares);
+    d_bfolds = reinterpret_cast<JumpFold *>(d_work + o_bfolds);
     items.clear();
     item_gen.clear();
     item_io.clear();
@@ -1487,10 +1540,10 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
         ji.masks = dw + o_masks + ji.masks;
         ji.states_out = (uint64_t)(uintptr_t)d_jstates + ji.states_out;
     }
-    for (auto &gr : mgroups) {
-        gr.planes += (uint64_t)(uintptr_t)d_jstates;
+    for (auto &gr : bgroups) {
+        gr.parts += (uint64_t)(uintptr_t)d_jstates;
         gr.out += (uint64_t)(uintptr_t)d_jstates;
-        gr.coef += dw + o_coef;
+        gr.coef += dw + o_bcoef;
     }
     if (!items.empty())
         memcpy(h_stage + o_items, items.data(), items.size() * sizeof(Item));
@@ -1502,10 +1555,18 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
         memcpy(h_stage + o_masks, mask_host.data(), mask_host.size() * 8);
     if (!jitems.empty())
         memcpy(h_stage + o_jitems, jitems.data(), jitems.size() * sizeof(JumpItem));
-    if (!mgroups.empty()) {
-        memcpy(h_stage + o_mgroups, mgroups.data(), mgroups.size() * sizeof(MJumpGroup));
-        memcpy(h_stage + o_mitems, mitems.data(), mitems.size() * sizeof(MJumpItem));
-        memcpy(h_stage + o_coef, coef_host.data(), coef_host.size() * 4);
+    if (!bgroups.empty()) {
+        memcpy(h_stage + o_bgroups, bgroups.data(), bgroups.size() * sizeof(JumpBlocks));
+        memcpy(h_stage + o_btiles, btiles.data(), btiles.size() * sizeof(JumpTile));
+        memcpy(h_stage + o_bshares, bshares.data(), bshares.size() * sizeof(JumpShare));
+        memcpy(h_stage + o_bfolds, bfolds.data(), bfolds.size() * sizeof(JumpFold));
+        uint32_t *cf = reinterpret_cast<uint32_t *>(h_stage + o_bcoef);
+        for (size_t i = 0; i < bcopies.size(); i++) {
+            const size_t room = (i + 1 < bcopies.size() ? bcopies[i + 1].at : bcoef_words) - bcopies[i].at;
+            const size_t m = std::min(room, bcopies[i].w->size());
+            memcpy(cf + bcopies[i].at, bcopies[i].w->data(), m * 4);
+            memset(cf + bcopies[i].at + m, 0, (room - m) * 4);
+        }
     }
     hip_check(hipMemcpyAsync(d_work, h_stage, work_bytes, hipMemcpyHostToDevice, opt.stream), "plan upload");
     if (!ev_upload)
@@ -1594,13 +1655,13 @@ void Plan::retarget(const std::vector<GenRef> &gens, hipStream_t s) {
     }
     for (size_t i = 0; i < jitems.size(); i++)
         jitems[i].state_in = (uint64_t)(uintptr_t)gens.at((size_t)jitem_gen[i]).state_in;
-    for (size_t i = 0; i < mgroups.size(); i++)
-        mgroups[i].state_in = (uint64_t)(uintptr_t)gens.at((size_t)mgroup_gen[i]).state_in;
+    for (size_t i = 0; i < bgroups.size(); i++)
+        bgroups[i].state_in = (uint64_t)(uintptr_t)gens.at((size_t)bgroup_gen[i]).state_in;
     wait_upload();
-    const size_t mb = mgroups.size() * sizeof(MJumpGroup);
-    if (mb) {
-        memcpy(h_stage + o_mgroups, mgroups.data(), mb);
-        hip_check(hipMemcpyAsync(d_work + o_mgroups, h_stage + o_mgroups, mb, hipMemcpyHostToDevice, s), "plan upload");
+    const size_t bb = bgroups.size() * sizeof(JumpBlocks);
+    if (bb) {
+        memcpy(h_stage + o_bgroups, bgroups.data(), bb);
+        hip_check(hipMemcpyAsync(d_work + o_bgroups, h_stage + o_bgroups, bb, hipMemcpyHostToDevice, s), "plan upload");
     }
     const size_t ib = items.size() * sizeof(Item), jb = jitems.size() * sizeof(JumpItem);
     if (ib) {
@@ -1663,16 +1724,14 @@ void Plan::run_launches(int part, int phase, hipStream_t s) {
     const auto &I = merged ? mlaunches : launches;
     const size_t iq = merged ? 2 * (launches.size() + jlaunches.size()) : 0;
     const size_t jq = iq + 2 * I.size();
-    if (part == 0 && !mgroups.empty()) {
-        // matrix-core jumps: the planes of the phase's groups, then the
-        // products by row-tile count
-        const MRange &R = mrange[merged ? 2 : phase];
-        if (R.g1 > R.g0) {
-            hip_check(launch_planes32(d_mgroups + R.g0, R.g1 - R.g0, ctx->d_params, s), "planes kernel launch");
-            for (int rt = 1; rt <= kMjRowTiles; rt++)
-                hip_check(launch_jump_mfma32(d_mgroups, d_mitems + R.i0[rt], R.i1[rt] - R.i0[rt], rt, s),
-                          "matrix-core jump launch");
-        }
+    // blocked jumps: round by round (a round reuses the partial windows'
+    // memory), the products of a class, then its folds
+    for (size_t k = 0; part == 0 && phase <= 0 && k < blaunches.size(); k++) {
+        const BLaunch &L = blaunches[k];
+        hip_check(launch_jump_tiles(L.bits, L.cls, d_bgroups, d_btiles, d_bshares + L.s0, L.s1 - L.s0, ctx->d_params, s),
+                  "blocked jump launch");
+        hip_check(launch_jump_folds(L.bits, L.cls, L.step, d_bgroups, d_bfolds + L.f0, L.f1 - L.f0, ctx->d_params, s),
+                  "jump fold launch");
     }
     for (size_t k = 0; part == 0 && k < J.size(); k++) {
         const Launch &L = J[k];
@@ -1837,8 +1896,10 @@ void Plan::free_device() {
     work_cap = jstates_cap = stage_cap = 0;
     d_items = nullptr;
     d_jitems = nullptr;
-    d_mgroups = nullptr;
-    d_mitems = nullptr;
+    d_bgroups = nullptr;
+    d_btiles = nullptr;
+    d_bshares = nullptr;
+    d_bfolds = nullptr;
 }
 
 Plan::~Plan() { free_device(); }
@@ -2640,14 +2701,7 @@ int mtgp_plan_stats(const mtgp_plan_t *p, int *items, int *launches, double *pla
         *items = (int)p->plan.items.size();
     if (launches) {  // kernel launches of one mtgp_plan_launch
         const Plan &P = p->plan;
-        int m = 0;
-        for (int ph = 0; ph < 3; ph++) {
-            if ((ph == 2) == P.two_phase() || P.mrange[ph].g1 <= P.mrange[ph].g0)
-                continue;
-            m++;
-            for (int rt = 1; rt <= kMjRowTiles; rt++)
-                m += P.mrange[ph].i1[rt] > P.mrange[ph].i0[rt];
-        }
+        const int m = 2 * (int)P.blaunches.size();
         *launches = m + (P.two_phase() ? (int)(P.launches.size() + P.jlaunches.size())
                                        : (int)(P.mlaunches.size() + P.mjlaunches.size()));
     }
@@ -2662,7 +2716,7 @@ int mtgp_plan_jump_stats(const mtgp_plan_t *p, int *jumps, int *matrix_jumps, in
     if (matrix_jumps)
         *matrix_jumps = p->plan.mjumps;
     if (matrix_groups)
-        *matrix_groups = (int)p->plan.mgroups.size();
+        *matrix_groups = p->plan.mgroups;
     return 0;
 }
 
@@ -2761,7 +2815,7 @@ int mtgp_genset_substreams(mtgp_genset_t *s, const void *base, const char *hex) 
     // Many substreams of an MTGP32 set: every one is a jump from the base,
     // so all of them are one matrix-core group (J^t for t < G from the
     // host, once per jump string).
-    const bool matrix = bits == 32 && c.jump_mfma_min > 0 && G - 1 >= c.jump_mfma_min;
+    const bool matrix = bits == 32 && c.jump_mfma_min > 0 && G - 1 >= std::max(256, c.jump_mfma_min);
     if (matrix && (!W.d || W.key != hex || !W.matrix)) {
         gf2::Poly J;
         if (!gf2::from_hex(hex, J))

@@ -17,6 +17,7 @@
 
 #include "common.hpp"
 #include "gf2x.hpp"
+#include "jump_blocks.hpp"
 
 namespace mtgp {
 
@@ -117,15 +118,15 @@ struct Context {
     // 16 measured best: one MTGP32-11213 stream (1017 jumps) 0.195 ms per
     // jump launch against 0.25 ms at 8; batches unchanged.
     int jump_max_parts = 16;
-    // A generator's jumps of one plan run on the matrix cores (MJumpGroup)
-    // when there are at least this many and its set is an MTGP32 one;
-    // 0 = never.  Measured on MI355X: one MTGP32-11213 stream of 2^24 + 2^24
-    // numbers (1016 jumps) 0.115 ms per jump launch against 0.19 ms; the
-    // 128-generator batch (45 jumps each) 0.53 against 0.51 ms, and the
-    // generation launch after a matrix-core jump launch runs 0.2 ms slower
-    // (the fp4 products draw the power the store-bound generation runs
-    // short of), so batches keep the batched jump kernel.
-    int jump_mfma_min = 256;
+    // A generator's jumps of one plan run in coefficient blocks on the matrix
+    // cores (jump_blocks.hpp) when there are at least this many, else by the
+    // word-XOR kernel; 0 = never.  The blocks were faster for every number
+    // of jumps measured (jump launches, blocks against word XORs): one
+    // MTGP32-11213 stream's 244 jumps 27 against 112 us, its 1008 jumps 58
+    // against 190 us; 976 MTGP64-23209 jumps 0.20 against 0.36 ms; 128
+    // generators of 45 MTGP32-11213 jumps 0.26 against 0.55 ms; 64 of 7
+    // MTGP64-44497 jumps 0.32 against 0.60 ms.
+    int jump_mfma_min = 1;
     struct Custom {
         DevParam rec;
         unsigned char sha1[20];
@@ -212,7 +213,6 @@ std::shared_ptr<gf2::Modulus> modulus_for(Context &c, int slot);
 // coefficient words: m[c * 64 + rho] bit q = coefficient of
 // x^(c * kJumpChunk + 64 q + rho).  And back.
 std::vector<uint16_t> jump_mask16(const std::vector<uint32_t> &words);
-std::vector<uint32_t> words_from_mask16(const std::vector<uint16_t> &m, int nwords);
 // Per-residue coefficient masks of up to kJumpBatch jumps (layout in
 // common.hpp), appended to `out`; returns the chunk count.
 int append_jump_masks16(const std::vector<const std::vector<uint16_t> *> &ms, std::vector<uint64_t> &out);
@@ -288,8 +288,7 @@ class JumpCache {
     struct Entry {
         std::shared_ptr<gf2::Modulus> mod;
         int words32 = 0;
-        std::vector<std::vector<uint16_t>> t1;  // [k] = x^(k cell) in mask form, k < B
-        std::vector<std::vector<uint32_t>> t1w; // the same as coefficient words
+        std::vector<std::vector<uint32_t>> t1w;  // [k] = x^(k cell) as coefficient words, k < B
         std::vector<gf2::Poly> t2p;              // [j] = x^(j B cell)
         std::vector<gf2::Poly> pow2;             // [i] = x^(2^i cell)
     };
@@ -357,21 +356,21 @@ struct Plan {
     std::vector<int32_t> item_gen, jitem_gen;
     std::vector<uint8_t> item_io;
     size_t o_items = 0, o_jitems = 0;  // their offsets in the workspace
-    // Matrix-core jumps: groups ordered by phase, items by (row tiles,
-    // phase); per phase (0, 1, 2 = merged) the group range and the item
-    // range of each row-tile count.  (A group holds all of a generator's
-    // jumps and counts as phase 0.)
-    std::vector<MJumpGroup> mgroups;
-    std::vector<MJumpItem> mitems;
-    std::vector<int32_t> mgroup_gen;
-    struct MRange {
-        int g0 = 0, g1 = 0;
-        int i0[kMjRowTiles + 1] = {}, i1[kMjRowTiles + 1] = {};
-    } mrange[3];
-    size_t o_mgroups = 0;
-    MJumpGroup *d_mgroups = nullptr;
-    MJumpItem *d_mitems = nullptr;
-    int mjumps = 0;  // jumps run on the matrix cores
+    // MTGP32 jumps run on the matrix cores, and their generators.
+    int mjumps = 0, mgroups = 0;
+    // Blocked matrix-core jumps (jump_blocks.hpp), rounds of launches in
+    // order: groups [g0, g1), product workgroups [s0, s1), folds [f0, f1).
+    struct BLaunch {
+        int bits = 0, cls = 0, step = 0, g0 = 0, g1 = 0, s0 = 0, s1 = 0, f0 = 0, f1 = 0;
+    };
+    std::vector<BLaunch> blaunches;
+    std::vector<JumpBlocks> bgroups;
+    std::vector<int32_t> bgroup_gen;
+    size_t o_bgroups = 0;
+    JumpBlocks *d_bgroups = nullptr;
+    JumpTile *d_btiles = nullptr;
+    JumpShare *d_bshares = nullptr;
+    JumpFold *d_bfolds = nullptr;
     hipEvent_t ev_upload = nullptr;    // the last upload from h_stage
     // Device copies: one grow-only workspace [items | segs | polys | masks |
     // jump items], the jumped-state arena and the work-queue counters.
