@@ -333,6 +333,7 @@ struct Plan {
         size_t dyn_lds;
         int phase;
         int layouts_ok;  // bit mask of the layouts allowed for these items
+        uint64_t numbers;  // generated or stepped over (generation launches)
     };
     Context *ctx = nullptr;
     // Start states of cells: 0 = jump inside the generation kernel
@@ -430,6 +431,9 @@ struct Plan {
     void launch_phase(int part, int phase, hipStream_t s);
     void run_launches(int part, int phase, hipStream_t s);  // phase -1: merged
     bool two_phase() const { return overlap && has_phase1; }
+    // Whether a short launch goes before a generation launch (see its
+    // definition).
+    bool settles(const Launch &L) const;
     void ensure_side();  // the side stream and fork/join events
     void set_overlap(bool on) {
         drop_graph();
