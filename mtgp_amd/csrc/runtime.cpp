@@ -749,52 +749,147 @@ constexpr int kAutoCacheMaxK = 2048;
 // Cells per block of an incremental polynomial chain on the host pool.
 constexpr size_t kChainMin = 32;
 
-// Partial windows of one round of blocked jumps, at most: they stay in the
-// 256 MB last-level cache between the products and the folds, and a plan of
-// any number of jumps needs no more memory for them.
-constexpr size_t kPartBytes = (size_t)128 << 20;
+// ----------------------------------------------------------- blocked jumps
+void JumpBlockList::clear() {
+    groups.clear();
+    tiles_.clear();
+    shares_.clear();
+    folds_.clear();
+    launches_.clear();
+    round_ = most_ = 0;
+    fresh_ = true;
+}
 
-// The tiles of one launch's groups [g0, g1) and the workgroups' shares of
-// them: kTilesPerCu workgroups per CU (the kernel's occupancy) with about the
-// same number of products each, so that one round of workgroups does the
-// launch and each makes its base's planes about once.  A tile of up to 32
-// columns does half the products of a wider one.
-constexpr int kTilesPerCu = 2;
-static void jb_tiles(const std::vector<JumpBlocks> &groups, int g0, int g1, int bits, int cus,
-                     std::vector<JumpTile> &tiles, std::vector<JumpShare> &shares) {
-    const int first = (int)tiles.size();
-    int64_t total = 0;
-    auto weight = [&](const JumpTile &t) { return groups[(size_t)t.group].ncols - t.c0 > 32 ? 2 : 1; };
-    for (int g = g0; g < g1; g++)
-        for (int plane = 0; plane < bits / 32; plane++)
-            for (int c0 = 0; c0 < groups[(size_t)g].ncols; c0 += kJbCols) {
-                tiles.push_back(JumpTile{g, c0, groups[(size_t)g].param, plane});
-                total += weight(tiles.back()) * (jb_plane_words(groups[(size_t)g].n) / kJbGroup);
+void JumpBlockList::add(const Context &c, int slot, uint64_t state_in, uint64_t coef, int ch, int nj, uint64_t out,
+                        uint64_t out_stride) {
+    const DevParam &D = c.param(slot);
+    const int cls = c.class_of(slot);
+    const size_t jbytes = (size_t)ch * (size_t)jb_part_words(D.bits, D.n) * 4;
+    for (int b0 = 0; b0 < nj;) {
+        size_t fit = round_ < kPartBytes ? (kPartBytes - round_) / jbytes : 0;
+        if (fit == 0) {
+            if (round_) {
+                fresh_ = true;
+                round_ = 0;
+                continue;
             }
-    const int64_t count = std::max<int64_t>(1, std::min<int64_t>(total, (int64_t)kTilesPerCu * cus));
-    JumpShare S{-1, 0, 0, 0, {}};
-    int64_t done = 0, made = 0;
-    for (int t = first; t < (int)tiles.size(); t++) {
-        const int w = weight(tiles[(size_t)t]), n = jb_plane_words(groups[(size_t)tiles[(size_t)t].group].n) / kJbGroup;
-        for (int at = 0; at < n;) {
-            if (S.tile0 < 0)
-                S.tile0 = t, S.g0 = at, S.first = tiles[(size_t)t];
-            // up to the end of the share: total * (made + 1) / count
-            const int64_t end = total * (made + 1) / count;
-            const int take = (int)std::min<int64_t>(n - at, std::max<int64_t>(1, (end - done + w - 1) / w));
-            at += take;
-            done += (int64_t)take * w;
-            S.tile1 = t, S.g1 = at;
-            if (done >= end) {
-                shares.push_back(S);
-                S.tile0 = -1;
-                while (made + 1 < count && done >= total * (made + 1) / count)
-                    made++;
+            fit = 1;
+        }
+        if (fresh_ || launches_.back().bits != D.bits || launches_.back().cls != cls) {
+            if (fresh_)
+                round_ = 0;
+            Launch L;
+            L.bits = D.bits;
+            L.cls = cls;
+            L.step = 1024;
+            L.g0 = L.g1 = (int)groups.size();
+            L.f0 = L.f1 = (int)folds_.size();
+            launches_.push_back(L);
+            fresh_ = false;
+        }
+        Launch &L = launches_.back();
+        const int m = (int)std::min<size_t>((size_t)(nj - b0), fit);
+        JumpBlocks gr{};
+        gr.state_in = state_in;
+        gr.coef = coef + (uint64_t)b0 * (uint64_t)ch * kJbWords * 4;
+        gr.parts = round_;
+        gr.out = out + (uint64_t)b0 * out_stride;
+        gr.out_stride = out_stride;
+        gr.ncols = m * ch;
+        gr.ch = ch;
+        gr.param = slot;
+        gr.n = D.n;
+        for (int b = 0; b < m; b++)
+            folds_.push_back(JumpFold{(int)groups.size(), b});
+        groups.push_back(gr);
+        L.step = std::min(L.step, jb_step(D.bits, cls, D.n, D.pos));
+        L.g1++;
+        L.f1 += m;
+        round_ += align256((size_t)m * jbytes);
+        most_ = std::max(most_, round_);
+        b0 += m;
+    }
+}
+
+// Each launch's shares: kSharesPerCu workgroups per CU (the kernel's
+// occupancy) with about the same number of products each, so that one round of
+// workgroups does the launch and each makes its base's planes about once.  A
+// tile of up to 32 columns does half the products of a wider one.
+void JumpBlockList::finish(int cus) {
+    constexpr int kSharesPerCu = 2;
+    auto weight = [&](const JumpTile &t) { return groups[(size_t)t.group].ncols - t.c0 > 32 ? 2 : 1; };
+    for (Launch &L : launches_) {
+        const int first = (int)tiles_.size();
+        int64_t total = 0;
+        for (int g = L.g0; g < L.g1; g++)
+            for (int plane = 0; plane < L.bits / 32; plane++)
+                for (int c0 = 0; c0 < groups[(size_t)g].ncols; c0 += kJbCols) {
+                    tiles_.push_back(JumpTile{g, c0, groups[(size_t)g].param, plane});
+                    total += weight(tiles_.back()) * (jb_plane_words(groups[(size_t)g].n) / kJbGroup);
+                }
+        const int64_t count = std::max<int64_t>(1, std::min<int64_t>(total, (int64_t)kSharesPerCu * cus));
+        L.s0 = (int)shares_.size();
+        JumpShare S{-1, 0, 0, 0, {}};
+        int64_t done = 0, made = 0;
+        for (int t = first; t < (int)tiles_.size(); t++) {
+            const JumpTile &T = tiles_[(size_t)t];
+            const int w = weight(T), n = jb_plane_words(groups[(size_t)T.group].n) / kJbGroup;
+            for (int at = 0; at < n;) {
+                if (S.tile0 < 0)
+                    S.tile0 = t, S.g0 = at, S.first = T;
+                // up to the end of the share: total * (made + 1) / count
+                const int64_t end = total * (made + 1) / count;
+                const int take = (int)std::min<int64_t>(n - at, std::max<int64_t>(1, (end - done + w - 1) / w));
+                at += take;
+                done += (int64_t)take * w;
+                S.tile1 = t, S.g1 = at;
+                if (done >= end) {
+                    shares_.push_back(S);
+                    S.tile0 = -1;
+                    while (made + 1 < count && done >= total * (made + 1) / count)
+                        made++;
+                }
             }
         }
+        if (S.tile0 >= 0)
+            shares_.push_back(S);
+        L.s1 = (int)shares_.size();
     }
-    if (S.tile0 >= 0)
-        shares.push_back(S);
+}
+
+void JumpBlockList::relocate(uint64_t coef, uint64_t parts, uint64_t out) {
+    for (JumpBlocks &g : groups) {
+        g.coef += coef;
+        g.parts += parts;
+        g.out += out;
+    }
+}
+
+size_t JumpBlockList::o_tiles() const { return align256(groups.size() * sizeof(JumpBlocks)); }
+size_t JumpBlockList::o_shares() const { return align256(o_tiles() + tiles_.size() * sizeof(JumpTile)); }
+size_t JumpBlockList::o_folds() const { return align256(o_shares() + shares_.size() * sizeof(JumpShare)); }
+size_t JumpBlockList::list_bytes() const { return align256(o_folds() + folds_.size() * sizeof(JumpFold)); }
+
+void JumpBlockList::write(char *h) const {
+    if (groups.empty())
+        return;
+    memcpy(h, groups.data(), groups.size() * sizeof(JumpBlocks));
+    memcpy(h + o_tiles(), tiles_.data(), tiles_.size() * sizeof(JumpTile));
+    memcpy(h + o_shares(), shares_.data(), shares_.size() * sizeof(JumpShare));
+    memcpy(h + o_folds(), folds_.data(), folds_.size() * sizeof(JumpFold));
+}
+
+void JumpBlockList::run(const Context &c, const char *d, hipStream_t s) const {
+    const JumpBlocks *g = reinterpret_cast<const JumpBlocks *>(d);
+    const JumpTile *t = reinterpret_cast<const JumpTile *>(d + o_tiles());
+    const JumpShare *sh = reinterpret_cast<const JumpShare *>(d + o_shares());
+    const JumpFold *f = reinterpret_cast<const JumpFold *>(d + o_folds());
+    for (const Launch &L : launches_) {
+        hip_check(launch_jump_tiles(L.bits, L.cls, g, t, sh + L.s0, L.s1 - L.s0, c.d_params, s),
+                  "blocked jump launch");
+        hip_check(launch_jump_folds(L.bits, L.cls, L.step, g, f + L.f0, L.f1 - L.f0, c.d_params, s),
+                  "jump fold launch");
+    }
 }
 
 GridModel grid_model_of(int bits, int cls, int mexp, int n) {
@@ -1303,99 +1398,41 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
         }
         arena_bytes += align256((size_t)P * nb * sbytes);
     }
-    // Blocked jumps: a generator's jumps as one JumpBlocks group, split where
-    // the partial windows of one round would outgrow kPartBytes.  Polynomials
-    // go up as they are, zero-padded to whole blocks; the jumped windows and
-    // (reused by every round) the partial windows lie in the arena.
-    bgroups.clear();
+    // Blocked jumps: polynomials go up as they are, zero-padded to whole
+    // blocks; the jumped windows and the partial windows lie in the arena.
+    blocks.clear();
     bgroup_gen.clear();
-    blaunches.clear();
     mjumps = mgroups = 0;
-    std::vector<JumpTile> btiles;
-    std::vector<JumpShare> bshares;
-    std::vector<JumpFold> bfolds;
     size_t bcoef_words = 0;
     struct BCopy {
         size_t at;
         const std::vector<uint32_t> *w;
     };
     std::vector<BCopy> bcopies;
-    {
-        std::stable_sort(bg.begin(), bg.end(), [&](const BGroup &a, const BGroup &b) {
-            return group_of(gens[(size_t)a.g]) < group_of(gens[(size_t)b.g]);
-        });
-        size_t round_bytes = 0, most = 0;
-        for (const BGroup &m : bg) {
-            const GenRef &ref = gens[(size_t)m.g];
-            if (ref.bits == 32) {
-                mgroups++;
-                mjumps += (int)m.cells.size();
-            }
-            const DevParam &D = c.param(ref.slot);
-            const int cls = c.class_of(ref.slot);
-            const int ch = jb_blocks(ref.mexp);
-            const size_t jbytes = (size_t)ch * (size_t)jb_part_words(ref.bits, ref.n) * 4;
-            const size_t sbytes = (size_t)ref.n * (size_t)(ref.bits / 8);
-            for (size_t b0 = 0; b0 < m.cells.size();) {
-                const size_t fit = round_bytes < kPartBytes ? (kPartBytes - round_bytes) / jbytes : 0;
-                const size_t nj = std::min(m.cells.size() - b0, std::max<size_t>(fit, round_bytes ? 0 : 1));
-                if (nj == 0) {
-                    round_bytes = 0;
-                    continue;
-                }
-                JumpBlocks gr{};
-                gr.state_in = (uint64_t)(uintptr_t)ref.state_in;
-                gr.coef = 4 * (uint64_t)bcoef_words;  // fixed up below
-                gr.parts = round_bytes;               // fixed up below
-                gr.out = arena_bytes;                 // fixed up below
-                gr.out_stride = sbytes;
-                gr.ncols = (int32_t)nj * ch;
-                gr.ch = ch;
-                gr.param = ref.slot;
-                gr.n = ref.n;
-                // a round's launches: one pair per (word size, class)
-                if (blaunches.empty() || round_bytes == 0 || blaunches.back().bits != ref.bits ||
-                    blaunches.back().cls != cls) {
-                    BLaunch L;
-                    L.bits = ref.bits;
-                    L.cls = cls;
-                    L.step = 1024;
-                    L.g0 = (int)bgroups.size();
-                    blaunches.push_back(L);
-                }
-                BLaunch &L = blaunches.back();
-                L.step = std::min(L.step, jb_step(ref.bits, cls, ref.n, D.pos));
-                L.f1 += (int)nj;
-                const int gi = (int)bgroups.size();
-                L.g1 = gi + 1;
-                for (size_t b = 0; b < nj; b++) {
-                    const size_t k = m.cells[b0 + b];
-                    slot_of[{m.g, k}] = std::make_tuple((uint64_t)(arena_bytes + b * sbytes), 1, (uint64_t)0);
-                    bcopies.push_back(BCopy{bcoef_words + b * (size_t)ch * kJbWords, words_of(m.g, k)});
-                    bfolds.push_back(JumpFold{gi, (int32_t)b});
-                }
-                bgroups.push_back(gr);
-                bgroup_gen.push_back(m.g);
-                bcoef_words += nj * (size_t)ch * kJbWords;
-                arena_bytes += align256(nj * sbytes);
-                round_bytes += align256(nj * jbytes);
-                most = std::max(most, round_bytes);
-                b0 += nj;
-            }
+    std::stable_sort(bg.begin(), bg.end(), [&](const BGroup &a, const BGroup &b) {
+        return group_of(gens[(size_t)a.g]) < group_of(gens[(size_t)b.g]);
+    });
+    for (const BGroup &m : bg) {
+        const GenRef &ref = gens[(size_t)m.g];
+        const int ch = jb_blocks(ref.mexp);
+        const size_t nj = m.cells.size(), sbytes = (size_t)ref.n * (size_t)(ref.bits / 8);
+        if (ref.bits == 32) {
+            mgroups++;
+            mjumps += (int)nj;
         }
-        const uint64_t parts_at = arena_bytes;
-        arena_bytes += most;
-        int f = 0;
-        for (BLaunch &L : blaunches) {
-            L.f0 = f;
-            f = L.f1 += f;
-            for (int gi = L.g0; gi < L.g1; gi++)
-                bgroups[(size_t)gi].parts += parts_at;
-            L.s0 = (int)bshares.size();
-            jb_tiles(bgroups, L.g0, L.g1, L.bits, c.cus, btiles, bshares);
-            L.s1 = (int)bshares.size();
+        blocks.add(c, ref.slot, (uint64_t)(uintptr_t)ref.state_in, 4 * (uint64_t)bcoef_words, ch, (int)nj, arena_bytes,
+                   sbytes);
+        bgroup_gen.resize(blocks.groups.size(), m.g);
+        for (size_t b = 0; b < nj; b++) {
+            slot_of[{m.g, m.cells[b]}] = std::make_tuple((uint64_t)(arena_bytes + b * sbytes), 1, (uint64_t)0);
+            bcopies.push_back(BCopy{bcoef_words + b * (size_t)ch * kJbWords, words_of(m.g, m.cells[b])});
         }
+        bcoef_words += nj * (size_t)ch * kJbWords;
+        arena_bytes += align256(nj * sbytes);
     }
+    blocks.finish(c.cus);
+    const size_t parts_at = arena_bytes;
+    arena_bytes += blocks.part_bytes();
     // Items, one per cell.
     std::vector<Item> list;
     std::vector<int> list_gen;
@@ -1496,15 +1533,12 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
     const size_t o_polys = align256(o_segs + segs.size() * sizeof(Segment));
     const size_t o_masks = align256(o_polys + poly_host.size() * 4);
     const size_t o_jitems = align256(o_masks + mask_host.size() * 8);
-    const size_t o_bgroups = align256(o_jitems + jitems.size() * sizeof(JumpItem));
-    const size_t o_btiles = align256(o_bgroups + bgroups.size() * sizeof(JumpBlocks));
-    const size_t o_bshares = align256(o_btiles + btiles.size() * sizeof(JumpTile));
-    const size_t o_bfolds = align256(o_bshares + bshares.size() * sizeof(JumpShare));
-    const size_t o_bcoef = align256(o_bfolds + bfolds.size() * sizeof(JumpFold));
+    const size_t o_blists = align256(o_jitems + jitems.size() * sizeof(JumpItem));
+    const size_t o_bcoef = o_blists + blocks.list_bytes();
     const size_t work_bytes = align256(o_bcoef + bcoef_words * 4);
     this->o_items = o_items;
     this->o_jitems = o_jitems;
-    this->o_bgroups = o_bgroups;
+    this->o_blists = o_blists;
     wait_upload();
     grow_device(d_work, work_cap, work_bytes, "hipMalloc plan workspace");
     grow_pinned(h_stage, stage_cap, work_bytes);
@@ -1517,10 +1551,6 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
     const uint64_t dw = (uint64_t)(uintptr_t)d_work;
     d_items = reinterpret_cast<Item *>(d_work + o_items);
     d_jitems = reinterpret_cast<JumpItem *>(d_work + o_jitems);
-    d_bgroups = reinterpret_cast<JumpBlocks *>(d_work + o_bgroups);
-    d_btiles = reinterpret_cast<JumpTile *>(d_work + o_btiles);
-    d_bshares = reinterpret_cast<JumpShare *>(d_work + o_bshares);
-    d_bfolds = reinterpret_cast<JumpFold *>(d_work + o_bfolds);
     items.clear();
     item_gen.clear();
     item_io.clear();
@@ -1540,11 +1570,7 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
         ji.masks = dw + o_masks + ji.masks;
         ji.states_out = (uint64_t)(uintptr_t)d_jstates + ji.states_out;
     }
-    for (auto &gr : bgroups) {
-        gr.parts += (uint64_t)(uintptr_t)d_jstates;
-        gr.out += (uint64_t)(uintptr_t)d_jstates;
-        gr.coef += dw + o_bcoef;
-    }
+    blocks.relocate(dw + o_bcoef, (uint64_t)(uintptr_t)d_jstates + parts_at, (uint64_t)(uintptr_t)d_jstates);
     if (!items.empty())
         memcpy(h_stage + o_items, items.data(), items.size() * sizeof(Item));
     if (!segs.empty())
@@ -1555,18 +1581,13 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
         memcpy(h_stage + o_masks, mask_host.data(), mask_host.size() * 8);
     if (!jitems.empty())
         memcpy(h_stage + o_jitems, jitems.data(), jitems.size() * sizeof(JumpItem));
-    if (!bgroups.empty()) {
-        memcpy(h_stage + o_bgroups, bgroups.data(), bgroups.size() * sizeof(JumpBlocks));
-        memcpy(h_stage + o_btiles, btiles.data(), btiles.size() * sizeof(JumpTile));
-        memcpy(h_stage + o_bshares, bshares.data(), bshares.size() * sizeof(JumpShare));
-        memcpy(h_stage + o_bfolds, bfolds.data(), bfolds.size() * sizeof(JumpFold));
-        uint32_t *cf = reinterpret_cast<uint32_t *>(h_stage + o_bcoef);
-        for (size_t i = 0; i < bcopies.size(); i++) {
-            const size_t room = (i + 1 < bcopies.size() ? bcopies[i + 1].at : bcoef_words) - bcopies[i].at;
-            const size_t m = std::min(room, bcopies[i].w->size());
-            memcpy(cf + bcopies[i].at, bcopies[i].w->data(), m * 4);
-            memset(cf + bcopies[i].at + m, 0, (room - m) * 4);
-        }
+    blocks.write(h_stage + o_blists);
+    for (size_t i = 0; i < bcopies.size(); i++) {
+        uint32_t *cf = reinterpret_cast<uint32_t *>(h_stage + o_bcoef) + bcopies[i].at;
+        const size_t room = (i + 1 < bcopies.size() ? bcopies[i + 1].at : bcoef_words) - bcopies[i].at;
+        const size_t m = std::min(room, bcopies[i].w->size());
+        memcpy(cf, bcopies[i].w->data(), m * 4);
+        memset(cf + m, 0, (room - m) * 4);
     }
     hip_check(hipMemcpyAsync(d_work, h_stage, work_bytes, hipMemcpyHostToDevice, opt.stream), "plan upload");
     if (!ev_upload)
@@ -1658,13 +1679,13 @@ void Plan::retarget(const std::vector<GenRef> &gens, hipStream_t s) {
     }
     for (size_t i = 0; i < jitems.size(); i++)
         jitems[i].state_in = (uint64_t)(uintptr_t)gens.at((size_t)jitem_gen[i]).state_in;
-    for (size_t i = 0; i < bgroups.size(); i++)
-        bgroups[i].state_in = (uint64_t)(uintptr_t)gens.at((size_t)bgroup_gen[i]).state_in;
+    for (size_t i = 0; i < blocks.groups.size(); i++)
+        blocks.groups[i].state_in = (uint64_t)(uintptr_t)gens.at((size_t)bgroup_gen[i]).state_in;
     wait_upload();
-    const size_t bb = bgroups.size() * sizeof(JumpBlocks);
+    const size_t bb = blocks.groups.size() * sizeof(JumpBlocks);
     if (bb) {
-        memcpy(h_stage + o_bgroups, bgroups.data(), bb);
-        hip_check(hipMemcpyAsync(d_work + o_bgroups, h_stage + o_bgroups, bb, hipMemcpyHostToDevice, s), "plan upload");
+        memcpy(h_stage + o_blists, blocks.groups.data(), bb);
+        hip_check(hipMemcpyAsync(d_work + o_blists, h_stage + o_blists, bb, hipMemcpyHostToDevice, s), "plan upload");
     }
     const size_t ib = items.size() * sizeof(Item), jb = jitems.size() * sizeof(JumpItem);
     if (ib) {
@@ -1727,15 +1748,8 @@ void Plan::run_launches(int part, int phase, hipStream_t s) {
     const auto &I = merged ? mlaunches : launches;
     const size_t iq = merged ? 2 * (launches.size() + jlaunches.size()) : 0;
     const size_t jq = iq + 2 * I.size();
-    // blocked jumps: round by round (a round reuses the partial windows'
-    // memory), the products of a class, then its folds
-    for (size_t k = 0; part == 0 && phase <= 0 && k < blaunches.size(); k++) {
-        const BLaunch &L = blaunches[k];
-        hip_check(launch_jump_tiles(L.bits, L.cls, d_bgroups, d_btiles, d_bshares + L.s0, L.s1 - L.s0, ctx->d_params, s),
-                  "blocked jump launch");
-        hip_check(launch_jump_folds(L.bits, L.cls, L.step, d_bgroups, d_bfolds + L.f0, L.f1 - L.f0, ctx->d_params, s),
-                  "jump fold launch");
-    }
+    if (part == 0 && phase <= 0)  // (blocked jumps of both phases run with phase 0)
+        blocks.run(*ctx, d_work + o_blists, s);
     for (size_t k = 0; part == 0 && k < J.size(); k++) {
         const Launch &L = J[k];
         if (!merged && L.phase != phase)
@@ -1916,10 +1930,6 @@ void Plan::free_device() {
     work_cap = jstates_cap = stage_cap = 0;
     d_items = nullptr;
     d_jitems = nullptr;
-    d_bgroups = nullptr;
-    d_btiles = nullptr;
-    d_bshares = nullptr;
-    d_bfolds = nullptr;
 }
 
 Plan::~Plan() { free_device(); }
@@ -2721,7 +2731,7 @@ int mtgp_plan_stats(const mtgp_plan_t *p, int *items, int *launches, double *pla
         *items = (int)p->plan.items.size();
     if (launches) {  // kernel launches of one mtgp_plan_launch
         const Plan &P = p->plan;
-        const int m = 2 * (int)P.blaunches.size();
+        const int m = P.blocks.launches();
         const auto &gen = P.two_phase() ? P.launches : P.mlaunches;
         *launches = m + (int)gen.size() + (int)(P.two_phase() ? P.jlaunches : P.mjlaunches).size();
         for (const auto &L : gen)
@@ -2820,6 +2830,102 @@ int mtgp_genset_jump(mtgp_genset_t *s, int g, const char *hex) {
     API_END(-1)
 }
 
+}  // extern "C"
+
+// The blocked work of mtgp_genset_substreams: substream t's window is the base
+// (substream 0's slot 0) jumped by J^t.
+//  - MTGP32 sets of more than kDirectSubstreams: every substream one jump from
+//    the base, J^t for t < G made on the host pool once per jump string, as
+//    the reference keeps its 4^k 3^162 table.
+//  - others: radix-4 levels, level m making t = a 4^m + j (a = 1..3, j < 4^m)
+//    as J^(a 4^m) applied to substream j -- the decomposition of t in powers of
+//    J the reference's substream samples use (openCL-sample/mtgp32-jump.cl:
+//    697-731); the host forms three polynomials per level.
+static void substream_blocks(mtgp_genset *s, const char *hex) {
+    constexpr int kDirectSubstreams = 256;
+    Context &c = *s->ctx;
+    auto &W = s->sub;
+    const int G = (int)s->bits.size(), slot = s->slot[0], mexp = s->mexp[0];
+    gf2::Poly J;
+    if (!gf2::from_hex(hex, J))
+        throw Error("jump string contains a non-hex character");
+    auto mod = modulus_for(c, slot);
+    J = mod->reduce_any(J);
+    const int ch = jb_blocks(mexp), words = ch * kJbWords;
+    std::vector<uint32_t> coef;
+    auto put = [&](size_t at, const gf2::Poly &p) {
+        const std::vector<uint32_t> w = gf2::to_words32(p, (mexp + 31) / 32);
+        memcpy(coef.data() + at, w.data(), std::min(w.size(), (size_t)words) * 4);
+    };
+    auto state = [&](long t) { return (uint64_t)(uintptr_t)s->state((int)t, 0); };
+    W.key.clear();
+    W.blocks.clear();
+    if (s->bits[0] == 32 && G > kDirectSubstreams) {
+        // chains of J products in blocks (a block starts from J^t0 by
+        // squarings)
+        coef.resize((size_t)(G - 1) * (size_t)words, 0u);
+        constexpr int kChain = 128;
+        parallel_for((G - 1 + kChain - 1) / kChain, [&](int blk) {
+            const int t0 = 1 + blk * kChain, t1 = std::min(G, t0 + kChain);
+            gf2::Poly cur, sq = J;
+            for (int e = t0; e; e >>= 1) {
+                if (e & 1)
+                    cur = cur.empty() ? sq : mod->mulmod(cur, sq);
+                if (e >> 1)
+                    sq = mod->sqrmod(sq);
+            }
+            for (int t = t0; t < t1; t++) {
+                if (t > t0)
+                    cur = mod->mulmod(cur, J);
+                put((size_t)(t - 1) * (size_t)words, cur);
+            }
+        });
+        W.blocks.add(c, slot, state(0), 0, ch, G - 1, state(1), state(1) - state(0));
+    } else {
+        gf2::Poly Jm = J;  // J^(4^m)
+        for (long p = 1; p < G; p *= 4) {
+            const size_t at = coef.size();
+            coef.resize(at + 3 * (size_t)words, 0u);
+            gf2::Poly Pa = Jm;
+            for (int a = 1; a < 4; a++) {
+                if (a > 1)
+                    Pa = mod->mulmod(Pa, Jm);
+                put(at + (size_t)(a - 1) * (size_t)words, Pa);
+            }
+            Jm = mod->mulmod(Pa, Jm);
+            W.blocks.depend();
+            for (long j = 0; j < p && p + j < G; j++)
+                W.blocks.add(c, slot, state(j), 4 * (uint64_t)at, ch, (int)std::min<long>(3, (G - 1 - j) / p), state(p + j),
+                             (uint64_t)p * (state(1) - state(0)));
+        }
+    }
+    W.blocks.finish(c.cus);
+    // workspace: [lists | coefficients | partial windows]
+    W.o_lists = 0;
+    const size_t o_coef = align256(W.blocks.list_bytes()), o_parts = align256(o_coef + coef.size() * 4);
+    const size_t need = std::max<size_t>(o_parts + W.blocks.part_bytes(), 256);
+    if (need > W.cap) {
+        if (W.d)
+            hip_check(hipFree(W.d), "hipFree");
+        W.d = nullptr;
+        W.cap = 0;
+        hip_check(hipMalloc((void **)&W.d, need), "hipMalloc substream workspace");
+        W.cap = need;
+    }
+    const uint64_t dw = (uint64_t)(uintptr_t)W.d;
+    W.blocks.relocate(dw + o_coef, dw + o_parts, 0);
+    std::vector<char> lists(o_coef);
+    W.blocks.write(lists.data());
+    hip_check(hipMemcpy(W.d, lists.data(), lists.size(), hipMemcpyHostToDevice), "hipMemcpy substream lists");
+    if (!coef.empty())
+        hip_check(hipMemcpy(W.d + o_coef, coef.data(), coef.size() * 4, hipMemcpyHostToDevice), "hipMemcpy coef");
+    W.first.clear();
+    W.blocked = true;
+    W.key = hex;
+}
+
+extern "C" {
+
 int mtgp_genset_substreams(mtgp_genset_t *s, const void *base, const char *hex) {
     API_BEGIN
     const int G = (int)s->bits.size();
@@ -2834,120 +2940,23 @@ int mtgp_genset_substreams(mtgp_genset_t *s, const void *base, const char *hex) 
     const size_t stride = align256(wbytes);
     const int occ = c.jump_blocks_per_cu[bits == 64][cls];
     auto &W = s->sub;
-    // Many substreams of an MTGP32 set: every one is a jump from the base,
-    // so all of them are one matrix-core group (J^t for t < G from the
-    // host, once per jump string).
-    const bool matrix = bits == 32 && c.jump_mfma_min > 0 && G - 1 >= std::max(256, c.jump_mfma_min);
-    if (matrix && (!W.d || W.key != hex || !W.matrix)) {
-        gf2::Poly J;
-        if (!gf2::from_hex(hex, J))
-            throw Error("jump string contains a non-hex character");
-        auto mod = modulus_for(c, s->slot[0]);
-        J = mod->reduce_any(J);
-        const int nj = G - 1, njp = (nj + 31) / 32 * 32;
-        const int kpad = mj_kpad(s->mexp[0]), wc = kpad / 32, pw = mj_pw(kpad, s->n[0]);
-        const int pwords = (s->mexp[0] + 31) / 32;
-        // coef[w * njp + (t - 1)] = word w of J^t, chains of J products in
-        // blocks on the host pool (a block starts from J^t0 by squarings)
-        std::vector<uint32_t> coef((size_t)wc * (size_t)njp, 0u);
-        constexpr int kBlock = 128;
-        parallel_for((nj + kBlock - 1) / kBlock, [&](int blk) {
-            const int t0 = 1 + blk * kBlock, t1 = std::min(G, t0 + kBlock);
-            gf2::Poly cur, sq = J;
-            for (int e = t0; e; e >>= 1) {
-                if (e & 1)
-                    cur = cur.empty() ? sq : mod->mulmod(cur, sq);
-                if (e >> 1)
-                    sq = mod->sqrmod(sq);
-            }
-            for (int t = t0; t < t1; t++) {
-                if (t > t0)
-                    cur = mod->mulmod(cur, J);
-                const std::vector<uint32_t> w = gf2::to_words32(cur, pwords);
-                for (size_t x = 0; x < w.size() && x < (size_t)wc; x++)
-                    coef[x * (size_t)njp + (size_t)(t - 1)] = w[x];
-            }
-        });
-        // workspace: [base | group | items | coef | planes | windows 1..G-1 | combine items]
-        std::vector<MJumpItem> mit[kMjRowTiles + 1];
-        for (int r0 = 0; r0 < nj; r0 += 32 * kMjRowTiles) {
-            const int rt = std::min(kMjRowTiles, (nj - r0 + 31) / 32);
-            for (int j0 = 0; j0 < s->n[0]; j0 += mj_words(rt))
-                mit[rt].push_back(MJumpItem{0, r0, j0, 0});
-        }
-        std::vector<MJumpItem> items;
-        for (int rt = 1; rt <= kMjRowTiles; rt++) {
-            W.mi_first[rt] = (int)items.size();
-            W.mi_count[rt] = (int)mit[rt].size();
-            items.insert(items.end(), mit[rt].begin(), mit[rt].end());
-        }
-        W.o_mgroup = stride;
-        W.o_mitems = align256(W.o_mgroup + sizeof(MJumpGroup));
-        const size_t o_coef = align256(W.o_mitems + items.size() * sizeof(MJumpItem));
-        const size_t o_planes = align256(o_coef + coef.size() * 4);
-        const size_t o_out = align256(o_planes + (size_t)pw * 32 * 4);
-        W.o_items = align256(o_out + (size_t)nj * wbytes);
-        const size_t need = W.o_items + (size_t)G * sizeof(JumpItem);
-        W.key.clear();
-        if (need > W.cap) {
-            if (W.d)
-                hip_check(hipFree(W.d), "hipFree");
-            W.d = nullptr;
-            W.cap = 0;
-            hip_check(hipMalloc((void **)&W.d, need), "hipMalloc substream workspace");
-            W.cap = need;
-        }
-        const uint64_t dw = (uint64_t)(uintptr_t)W.d;
-        MJumpGroup gr{};
-        gr.state_in = dw;
-        gr.in_parts = 1;
-        gr.planes = dw + o_planes;
-        gr.coef = dw + o_coef;
-        gr.out = dw + o_out;
-        gr.out_stride = wbytes;
-        gr.nj = nj;
-        gr.njp = njp;
-        gr.kpad = kpad;
-        gr.pw = pw;
-        gr.param = s->slot[0];
-        gr.n = s->n[0];
-        // combine: substream t's window (the base for t = 0) into slot 0
-        std::vector<JumpItem> copies((size_t)G);
-        for (int t = 0; t < G; t++) {
-            JumpItem &ji = copies[(size_t)t];
-            ji.state_in = t ? dw + o_out + (uint64_t)(t - 1) * wbytes : dw;
-            ji.in_parts = 1;
-            ji.states_out = (uint64_t)(uintptr_t)s->state(t, 0);
-            ji.state_bytes = (int32_t)wbytes;
-        }
-        W.combine_first = 0;
-        W.combine_count = G;
-        hip_check(hipMemcpy(W.d + W.o_mgroup, &gr, sizeof gr, hipMemcpyHostToDevice), "hipMemcpy group");
-        hip_check(hipMemcpy(W.d + W.o_mitems, items.data(), items.size() * sizeof(MJumpItem), hipMemcpyHostToDevice),
-                  "hipMemcpy items");
-        hip_check(hipMemcpy(W.d + o_coef, coef.data(), coef.size() * 4, hipMemcpyHostToDevice), "hipMemcpy coef");
-        hip_check(hipMemcpy(W.d + W.o_items, copies.data(), copies.size() * sizeof(JumpItem), hipMemcpyHostToDevice),
-                  "hipMemcpy combine items");
-        W.first.clear();
-        W.matrix = true;
-        W.key = hex;
-    }
-    if (matrix) {
-        hip_check(hipMemcpy(W.d, base, wbytes, hipMemcpyHostToDevice), "hipMemcpy base");
-        const MJumpGroup *d_group = reinterpret_cast<const MJumpGroup *>(W.d + W.o_mgroup);
-        const MJumpItem *d_mitems = reinterpret_cast<const MJumpItem *>(W.d + W.o_mitems);
-        hip_check(launch_planes32(d_group, 1, c.d_params, 0), "planes kernel launch");
-        for (int rt = 1; rt <= kMjRowTiles; rt++)
-            hip_check(launch_jump_mfma32(d_group, d_mitems + W.mi_first[rt], W.mi_count[rt], rt, 0),
-                      "matrix-core jump launch");
-        hip_check(launch_combine(reinterpret_cast<const JumpItem *>(W.d + W.o_items), G, 0), "combine launch");
+    // Matrix cores on: blocked jumps, straight into the set's slots 0.
+    const bool blocked = c.jump_mfma_min > 0;
+    if (blocked) {
+        if (!W.d || W.key != hex || !W.blocked)
+            substream_blocks(s, hex);
+        std::lock_guard<std::mutex> lk(c.jump_mu);  // the pinned staging buffer
+        grow_pinned(c.jump_h, c.jump_hcap, wbytes);
+        memcpy(c.jump_h, base, wbytes);
+        hip_check(hipMemcpyAsync(s->state(0, 0), c.jump_h, wbytes, hipMemcpyHostToDevice, nullptr), "hipMemcpyAsync base");
+        W.blocks.run(c, W.d + W.o_lists, nullptr);
         hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");
         for (int g = 0; g < G; g++)
             s->set_cur(g, 0);
         return 0;
     }
-    if (!W.d || W.key != hex || W.matrix) {
-        W.matrix = false;
+    if (!W.d || W.key != hex || W.blocked) {
+        W.blocked = false;
         // Substream t = J^t applied to the base, built on the device in
         // radix-4 levels: level m makes t = a 4^m + j (a = 1..3, j < 4^m)
         // as J^(a 4^m) applied to substream j -- the decomposition of t in

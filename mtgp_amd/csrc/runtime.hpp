@@ -308,6 +308,53 @@ struct PlanOptions {
     int overlap = -1;              // two-phase launch (see Plan): 1 on, 0 off, -1 default
 };
 
+// Jumps in coefficient blocks (jump_blocks.hpp): the groups, tiles, shares
+// and folds of a sequence of launches.  The partial windows of one round of
+// launches take at most kPartBytes (they then stay in the 256 MB last-level
+// cache between the products and the folds, and any number of jumps needs no
+// more memory for them); the next round reuses their place.
+class JumpBlockList {
+  public:
+    static constexpr size_t kPartBytes = (size_t)128 << 20;
+    void clear();
+    bool empty() const { return groups.empty(); }
+    // Appends nj jumps of the window at state_in: polynomials of ch blocks
+    // each at coef (ch * kJbWords words per jump), jump b's window to out +
+    // b * out_stride.  May split them into several groups.
+    void add(const Context &c, int slot, uint64_t state_in, uint64_t coef, int ch, int nj, uint64_t out,
+             uint64_t out_stride);
+    // The jumps added from here on read windows that those before write.
+    void depend() { fresh_ = true; }
+    // After the last add: makes the tiles and shares.  The partial windows
+    // need part_bytes() at `parts` (finish adds it to the groups).
+    void finish(int cus);
+    size_t part_bytes() const { return most_; }
+    // Added to every group's addresses of the kind.
+    void relocate(uint64_t coef, uint64_t parts, uint64_t out);
+    // The device lists: their size, and their bytes to an upload buffer.
+    size_t list_bytes() const;
+    void write(char *h) const;
+    // Every launch, from the lists at d_lists.
+    void run(const Context &c, const char *d_lists, hipStream_t s) const;
+    int launches() const { return 2 * (int)launches_.size(); }
+    std::vector<JumpBlocks> groups;
+
+  private:
+    // Groups [g0, g1), product workgroups [s0, s1), folds [f0, f1).
+    struct Launch {
+        int bits = 0, cls = 0, step = 0, g0 = 0, g1 = 0, s0 = 0, s1 = 0, f0 = 0, f1 = 0;
+    };
+    size_t o_tiles() const;
+    size_t o_shares() const;
+    size_t o_folds() const;
+    std::vector<JumpTile> tiles_;
+    std::vector<JumpShare> shares_;
+    std::vector<JumpFold> folds_;
+    std::vector<Launch> launches_;
+    size_t round_ = 0, most_ = 0;
+    bool fresh_ = true;
+};
+
 // A list of device Items plus the launches that run them.
 //
 // Each generator's requests occupy consecutive positions of its stream
@@ -359,19 +406,11 @@ struct Plan {
     size_t o_items = 0, o_jitems = 0;  // their offsets in the workspace
     // MTGP32 jumps run on the matrix cores, and their generators.
     int mjumps = 0, mgroups = 0;
-    // Blocked matrix-core jumps (jump_blocks.hpp), rounds of launches in
-    // order: groups [g0, g1), product workgroups [s0, s1), folds [f0, f1).
-    struct BLaunch {
-        int bits = 0, cls = 0, step = 0, g0 = 0, g1 = 0, s0 = 0, s1 = 0, f0 = 0, f1 = 0;
-    };
-    std::vector<BLaunch> blaunches;
-    std::vector<JumpBlocks> bgroups;
+    // Blocked matrix-core jumps, their lists at o_blists in the workspace, and
+    // the generator of each of their groups.
+    JumpBlockList blocks;
     std::vector<int32_t> bgroup_gen;
-    size_t o_bgroups = 0;
-    JumpBlocks *d_bgroups = nullptr;
-    JumpTile *d_btiles = nullptr;
-    JumpShare *d_bshares = nullptr;
-    JumpFold *d_bfolds = nullptr;
+    size_t o_blists = 0;
     hipEvent_t ev_upload = nullptr;    // the last upload from h_stage
     // Device copies: one grow-only workspace [items | segs | polys | masks |
     // jump items], the jumped-state arena and the work-queue counters.
@@ -490,12 +529,10 @@ struct mtgp_genset {
         std::vector<int> first;  // jump launches: items [first[k], first[k+1])
         int combine_first = 0, combine_count = 0;
         size_t o_items = 0, o_queue = 0;
-        // Matrix-core variant: one MJumpGroup of every substream from the
-        // base, its items by row-tile count [mi_first[rt], mi_first[rt] +
-        // mi_count[rt]) at o_mitems.
-        bool matrix = false;
-        size_t o_mgroup = 0, o_mitems = 0;
-        int mi_first[mtgp::kMjRowTiles + 1] = {}, mi_count[mtgp::kMjRowTiles + 1] = {};
+        // Blocked variant: its launches, their lists at o_lists.
+        bool blocked = false;
+        mtgp::JumpBlockList blocks;
+        size_t o_lists = 0;
     } sub;
     // mtgp_genset_generate's plan, reused so that repeated calls allocate
     // nothing once their sizes have been seen (calls on one set serialise).
