@@ -1969,6 +1969,55 @@ struct mtgp_plan {
     }
 };
 
+// One jump in coefficient blocks: the block lists, coefficients and (host_io)
+// the window go up in one copy to the context's workspace [lists |
+// coefficients | window in | partial windows | window out], two launches, the
+// window back.  False (nothing done) when the partial windows of a very long
+// polynomial would outgrow a round's memory.
+static bool device_jump_blocks(Context &c, int slot, int bits, int mexp, const void *in, void *out,
+                               const std::vector<uint32_t> &words, bool host_io) {
+    const int n = state_words(bits, mexp);
+    const size_t wbytes = (size_t)n * (size_t)(bits / 8);
+    size_t top = words.size();
+    while (top > 1 && words[top - 1] == 0)
+        top--;
+    const size_t blocks = (top + kJbWords - 1) / kJbWords;
+    if (blocks * (size_t)jb_part_words(bits, n) * 4 > JumpBlockList::kPartBytes)
+        return false;
+    JumpBlockList L;
+    L.add(c, slot, host_io ? 0 : (uint64_t)(uintptr_t)in, 0, (int)blocks, 1, host_io ? 0 : (uint64_t)(uintptr_t)out,
+          wbytes);
+    L.finish(c.cus);
+    const size_t o_coef = L.list_bytes();
+    const size_t o_in = o_coef + align256(blocks * kJbWords * 4);
+    const size_t o_parts = o_in + align256(wbytes);
+    const size_t o_out = o_parts + L.part_bytes();
+    const size_t need = o_out + align256(wbytes);
+    std::lock_guard<std::mutex> lk(c.jump_mu);
+    grow_device(c.jump_d, c.jump_dcap, need, "hipMalloc jump workspace");
+    grow_pinned(c.jump_h, c.jump_hcap, need);
+    char *d = c.jump_d, *h = c.jump_h;
+    const uint64_t dw = (uint64_t)(uintptr_t)d;
+    L.relocate(dw + o_coef, dw + o_parts, host_io ? dw + o_out : 0);
+    if (host_io)
+        L.groups[0].state_in = dw + o_in;
+    L.write(h);
+    memset(h + o_coef, 0, blocks * kJbWords * 4);
+    memcpy(h + o_coef, words.data(), top * 4);
+    if (host_io)
+        memcpy(h + o_in, in, wbytes);
+    hip_check(hipMemcpyAsync(d, h, host_io ? o_in + wbytes : o_in, hipMemcpyHostToDevice, nullptr),
+              "hipMemcpyAsync jump workspace");
+    L.run(c, d, nullptr);
+    if (host_io)
+        hip_check(hipMemcpyAsync(h + o_out, d + o_out, wbytes, hipMemcpyDeviceToHost, nullptr),
+                  "hipMemcpyAsync jumped window");
+    hip_check(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
+    if (host_io)
+        memcpy(out, h + o_out, wbytes);
+    return true;
+}
+
 // Applies a jump polynomial (hex) to device window `in`, result in `out`.
 // A single jump on one wave is latency-bound (the fold of every chunk of
 // the polynomial in sequence), so it is split into partial jumps over chunk
@@ -1989,6 +2038,8 @@ static void device_jump(Context &c, int slot, int bits, int mexp, const void *in
     // Applied literally, as mtgp32_fast_jump does: every coefficient of the
     // string, whatever its degree (the kernel runs the sequence that far).
     const std::vector<uint32_t> words = gf2::to_words32(P, std::max<int>(1, (int)((strlen(hex) * 4 + 31) / 32)));
+    if (c.jump_mfma_min == 1 && device_jump_blocks(c, slot, bits, mexp, in, out, words, host_io))
+        return;
     std::vector<uint64_t> masks;
     const int chunks = append_jump_masks({&words}, masks);
     const size_t id_off = masks.size();
@@ -2940,8 +2991,8 @@ int mtgp_genset_substreams(mtgp_genset_t *s, const void *base, const char *hex) 
     const size_t stride = align256(wbytes);
     const int occ = c.jump_blocks_per_cu[bits == 64][cls];
     auto &W = s->sub;
-    // Matrix cores on: blocked jumps, straight into the set's slots 0.
-    const bool blocked = c.jump_mfma_min > 0;
+    // Blocked jumps, straight into the set's slots 0.
+    const bool blocked = c.jump_mfma_min > 0 && std::max(1, G - 1) >= c.jump_mfma_min;
     if (blocked) {
         if (!W.d || W.key != hex || !W.blocked)
             substream_blocks(s, hex);

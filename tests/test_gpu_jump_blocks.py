@@ -68,3 +68,37 @@ def test_substreams(mtgp, oracle, bits, mexp, count):
                 got, mask = gs.state(t), w.dtype.type(p.mask)
                 assert (got[1:] == w[1:]).all() and got[0] & mask == w[0] & mask, t
             w = oracle.jump(p, w, js)
+
+
+@pytest.mark.parametrize("bits,mexp", [(32, 11213), (32, 44497), (64, 23209), (64, 110503)])
+def test_single_jumps(mtgp, oracle, bits, mexp):
+    """Polynomials at the edges of the blocks, applied to a host generator and
+    to a device set: the zero polynomial, 1, x, the last coefficient of a
+    block and the first of the next, one block and a word, dense ones, and one
+    of higher degree than the set's."""
+    print("blocked jumps: single jumps of MTGP%d-%d" % (bits, mexp), flush=True)
+    p = oracle.params(bits, mexp, 6)
+    rng = np.random.default_rng(mexp)
+
+    def hexs(coeffs):
+        # four coefficients per character, the lowest ones first
+        v = np.zeros(max(list(coeffs) + [0]) // 4 + 1, int)
+        for k in coeffs:
+            v[k // 4] |= 1 << (k % 4)
+        return "".join("%x" % q for q in v)
+
+    dense = [k for k in range(mexp) if rng.random() < 0.5]
+    polys = [[], [0], [1], [1023], [1024], [0, 1023, 1024, 1055], dense, dense[:1000] + [mexp + 3000]]
+    G = mtgp.Generator32 if bits == 32 else mtgp.Generator64
+    for k, cs in enumerate(polys):
+        s = hexs(cs)
+        g = G(mexp, 6, seed=5 + k)
+        gs = mtgp.GenSet([(bits, mexp, 6)])
+        gs.init_seed([5 + k])
+        w = oracle.init_state(p, 5 + k)
+        assert (g.window() == w).all()
+        want = oracle.jump(p, w, s)
+        g.fast_jump(s)
+        assert (g.window() == want).all(), k
+        gs.jump(0, s)
+        assert (gs.state(0) == want).all(), k
