@@ -23,8 +23,13 @@
 //    scanning c's set bits with scalar instructions.  This is the same
 //    state as the reference's mtgp32_fast_jump (mtgp32-fast-jump.c:51-79).
 //  * Work distribution: workgroup g starts with Item g, then takes further
-//    Items from an atomic counter; the last workgroup to finish resets the
-//    counter pair, so launches need no memset and are graph-capturable.
+//    Items from an atomic counter, which the last claim resets, so launches
+//    need no memset and are graph-capturable.  A launch with a workgroup for
+//    every Item makes no claims: the atomics of all workgroups on one address
+//    run one after the other, about 10 ns each, and two per workgroup (a claim
+//    and a count of the finished) were most of a short launch: 1024 cells of
+//    4 steps 33.6 us, without them 6.3; one stream of 2^24 numbers in 1009
+//    cells 44.8 -> 22.3 us; 5*10^6 MTGP64 numbers in 977 cells 35.9 -> 12.5.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -52,6 +57,17 @@ constexpr int kWave = 64;
 constexpr int kStep = 256;  // words per wave step (4 per lane)
 
 __device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// Takes the next Item past the first gridDim.x from the launch's counter
+// (queue[0], zero before the launch).  Every workgroup ends with one claim past
+// the list, so a launch makes exactly n_items claims and the one that gets the
+// last number leaves the counter at zero again.
+__device__ __forceinline__ uint32_t claim(uint32_t *queue, int n_items) {
+    const uint32_t next = atomicAdd(&queue[0], 1u);
+    if (next == (uint32_t)n_items - 1)
+        atomicExch(&queue[0], 0u);
+    return next;
+}
 
 // Orders the workgroup's LDS accesses across steps (a barrier of one wave,
 // or of the two waves of a layout-2 cell).
@@ -499,26 +515,21 @@ __global__ __launch_bounds__(64 * W) void mtgp32_items_kernel(const Item *__rest
         if (state_out)
             for (int j = l; j < p.n; j += T)
                 state_out[j] = buf[b + j];
+        if ((uint32_t)n_items <= gridDim.x)
+            return;  // one item per workgroup: nothing to claim (see the file header)
         wave_sync();
         if constexpr (W == 1) {
             uint32_t next = 0;
             if (l == 0)
-                next = atomicAdd(&queue[0], 1u);
+                next = claim(queue, n_items);
             it = gridDim.x + uniform(__shfl(next, 0));
         } else {
             // One claim per workgroup, handed to every wave through LDS.
             if (l == 0)
-                next_item = atomicAdd(&queue[0], 1u);
+                next_item = claim(queue, n_items);
             wave_sync();
             it = gridDim.x + uniform(next_item);
             wave_sync();
-        }
-    }
-    if (l == 0) {
-        __threadfence();
-        if (atomicAdd(&queue[1], 1u) == gridDim.x - 1) {
-            atomicExch(&queue[0], 0u);
-            atomicExch(&queue[1], 0u);
         }
     }
 }
@@ -954,26 +965,21 @@ __global__ __launch_bounds__(64 * WV) void mtgp64_items_kernel(const Item *__res
         if (state_out)
             for (int j = l; j < p.n; j += T)
                 state_out[j] = ((uint64_t)bh[b + j] << 32) | bl[b + j];
+        if ((uint32_t)n_items <= gridDim.x)
+            return;  // one item per workgroup: nothing to claim (see the file header)
         wave_sync();
         if constexpr (WV == 1) {
             uint32_t next = 0;
             if (l == 0)
-                next = atomicAdd(&queue[0], 1u);
+                next = claim(queue, n_items);
             it = gridDim.x + uniform(__shfl(next, 0));
         } else {
             // One claim per workgroup, handed to every wave through LDS.
             if (l == 0)
-                next_item = atomicAdd(&queue[0], 1u);
+                next_item = claim(queue, n_items);
             wave_sync();
             it = gridDim.x + uniform(next_item);
             wave_sync();
-        }
-    }
-    if (l == 0) {
-        __threadfence();
-        if (atomicAdd(&queue[1], 1u) == gridDim.x - 1) {
-            atomicExch(&queue[0], 0u);
-            atomicExch(&queue[1], 0u);
         }
     }
 }
@@ -1104,18 +1110,13 @@ __global__ __launch_bounds__(64) void mtgp32_jump_kernel(const JumpItem *__restr
                         o[l + kWave * m] = acc[b][m];
             }
         }
+        if ((uint32_t)n_items <= gridDim.x)
+            return;
         wave_sync();
         uint32_t next = 0;
         if (l == 0)
-            next = atomicAdd(&queue[0], 1u);
+            next = claim(queue, n_items);
         it = gridDim.x + uniform(__shfl(next, 0));
-    }
-    if (l == 0) {
-        __threadfence();
-        if (atomicAdd(&queue[1], 1u) == gridDim.x - 1) {
-            atomicExch(&queue[0], 0u);
-            atomicExch(&queue[1], 0u);
-        }
     }
 }
 
@@ -1196,18 +1197,13 @@ __global__ __launch_bounds__(64) void mtgp64_jump_kernel(const JumpItem *__restr
                         o[l + kWave * m] = ((uint64_t)ah[b][m] << 32) | al[b][m];
             }
         }
+        if ((uint32_t)n_items <= gridDim.x)
+            return;
         wave_sync();
         uint32_t next = 0;
         if (l == 0)
-            next = atomicAdd(&queue[0], 1u);
+            next = claim(queue, n_items);
         it = gridDim.x + uniform(__shfl(next, 0));
-    }
-    if (l == 0) {
-        __threadfence();
-        if (atomicAdd(&queue[1], 1u) == gridDim.x - 1) {
-            atomicExch(&queue[0], 0u);
-            atomicExch(&queue[1], 0u);
-        }
     }
 }
 

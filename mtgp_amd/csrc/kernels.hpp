@@ -34,8 +34,8 @@ int kernel_threads(int bits, int cls, int layout);
 // Its template name, as profilers print it (e.g. mtgp32_items_kernel<351,3,1,1,4>).
 std::string kernel_name(int bits, int cls, int layout);
 // Runs items[0, n_items) (device array, all of word size `bits` and class
-// <= cls) with `grid` persistent workgroups.  `queue` is a device pair of
-// uint32_t counters that is zero on entry and zero again on exit.
+// <= cls) with `grid` persistent workgroups.  `queue` is a device uint32_t
+// counter that is zero on entry and zero again on exit.
 // `dyn_lds` bytes of unused dynamic LDS per workgroup cap how many
 // workgroups a CU holds at once (even placement of one-item-per-wave grids).
 hipError_t launch_items(int bits, int cls, int layout, const Item *items, int n_items, const DevParam *params,
