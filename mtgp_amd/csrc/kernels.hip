@@ -456,7 +456,7 @@ template <int NMAX, int K, int LAYOUT, int W = 1, int WPL = 4>
 __global__ __launch_bounds__(64 * W) void mtgp32_items_kernel(const Item *__restrict__ items, int n_items,
                                                               const DevParam *__restrict__ params,
                                                               uint32_t *__restrict__ queue) {
-    static_assert(WPL == 4 || (W > 1 && WPL == 2), "words per lane");
+    static_assert(WPL == 4 || (W > 1 && WPL == 2) || (W == 4 && WPL == 1), "words per lane");
     constexpr int T = kWave * W;
     constexpr int NJ = (NMAX + T - 1) / T;
     constexpr int NBUF = K * T * WPL + T * NJ + T;
@@ -1212,6 +1212,15 @@ __global__ __launch_bounds__(64) void mtgp64_jump_kernel(const JumpItem *__restr
 #define MTGP_RELOC_STEPS 3
 #endif
 constexpr int kK = MTGP_RELOC_STEPS;
+// The same for the cells of one word per lane (layout 3 of the smallest
+// classes), whose every step is one short chain of LDS reads, the two table
+// lookups, a write and a barrier: about 175 ns whatever the stores do, so
+// these cells are for launches too small to fill the chip (one MTGP32-11213
+// stream of 2^24 words in 512 cells: two words per lane and two waves 36.3
+// us, one word and four waves 28.3; 2017 cells 17.2 and 17.4).  4, 8, 12 steps:
+// 256 cells 53.1, 50.9, 50.0 us; 12 would leave MTGP64 cells room
+// for five workgroups per CU instead of seven.
+constexpr int kKLatency = 8;
 
 // Largest state of the 64-bit narrow class (128-word steps).
 constexpr int kNarrowN = 176;
@@ -1226,10 +1235,13 @@ template <int NMAX, int LAYOUT>
 struct KernelOf<32, NMAX, LAYOUT, 4> {
     static constexpr int waves = LAYOUT == 3 ? 4 : LAYOUT == 2 ? 2 : 1;
     static constexpr int step_layout = LAYOUT >= 2 ? 1 : LAYOUT;
-    static constexpr int wpl = (LAYOUT == 2 && NMAX <= 351) || (LAYOUT == 3 && NMAX <= 726) ? 2 : 4;
-    static constexpr auto fn = mtgp32_items_kernel<NMAX, kK, step_layout, waves, wpl>;
+    static constexpr int wpl = LAYOUT == 3 && NMAX <= 351                                  ? 1
+                               : (LAYOUT == 2 && NMAX <= 351) || (LAYOUT == 3 && NMAX <= 726) ? 2
+                                                                                              : 4;
+    static constexpr int k = wpl == 1 ? kKLatency : kK;
+    static constexpr auto fn = mtgp32_items_kernel<NMAX, k, step_layout, waves, wpl>;
     static std::string name() {
-        return "mtgp32_items_kernel<" + std::to_string(NMAX) + "," + std::to_string(kK) + "," +
+        return "mtgp32_items_kernel<" + std::to_string(NMAX) + "," + std::to_string(k) + "," +
                std::to_string(step_layout) + "," + std::to_string(waves) + "," + std::to_string(wpl) + ">";
     }
 };
@@ -1237,10 +1249,13 @@ template <int NMAX, int LAYOUT, int WPL>
 struct KernelOf<64, NMAX, LAYOUT, WPL> {
     static constexpr int waves = LAYOUT == 3 ? 4 : LAYOUT == 2 ? 2 : 1;
     static constexpr int step_layout = LAYOUT >= 2 ? 1 : LAYOUT;
-    static constexpr int wpl = (LAYOUT == 2 && NMAX <= 363) || (LAYOUT == 3 && NMAX <= 696) ? 2 : WPL;
-    static constexpr auto fn = mtgp64_items_kernel<NMAX, kK, step_layout, wpl, waves>;
+    static constexpr int wpl = LAYOUT == 3 && NMAX <= 363                                  ? 1
+                               : (LAYOUT == 2 && NMAX <= 363) || (LAYOUT == 3 && NMAX <= 696) ? 2
+                                                                                              : WPL;
+    static constexpr int k = wpl == 1 ? kKLatency : kK;
+    static constexpr auto fn = mtgp64_items_kernel<NMAX, k, step_layout, wpl, waves>;
     static std::string name() {
-        return "mtgp64_items_kernel<" + std::to_string(NMAX) + "," + std::to_string(kK) + "," +
+        return "mtgp64_items_kernel<" + std::to_string(NMAX) + "," + std::to_string(k) + "," +
                std::to_string(step_layout) + "," + std::to_string(wpl) + "," + std::to_string(waves) + ">";
     }
 };
@@ -1265,8 +1280,8 @@ auto with_kernel(int bits, int cls, int layout, F &&f) {
 #define N_OF(B, c) ((B) == 32 ? ((c) == 0 ? 351 : (c) == 1 ? 726 : 1391) : ((c) == 0 ? 363 : (c) == 1 ? 696 : 1727))
     MTGP_CASE(32, 351, 0) MTGP_CASE(32, 351, 1) MTGP_CASE(32, 726, 0) MTGP_CASE(32, 726, 1)
     MTGP_CASE(32, 1391, 0) MTGP_CASE(32, 1391, 1) MTGP_CASE(32, 351, 2) MTGP_CASE(32, 726, 2)
-    MTGP_CASE(32, 1391, 2) MTGP_CASE(32, 726, 3) MTGP_CASE(32, 1391, 3) MTGP_CASE(64, 363, 0) MTGP_CASE(64, 363, 1)
-    MTGP_CASE(64, 363, 2)
+    MTGP_CASE(32, 1391, 2) MTGP_CASE(32, 351, 3) MTGP_CASE(32, 726, 3) MTGP_CASE(32, 1391, 3)
+    MTGP_CASE(64, 363, 0) MTGP_CASE(64, 363, 1) MTGP_CASE(64, 363, 2) MTGP_CASE(64, 363, 3)
     MTGP_CASE(64, 696, 0) MTGP_CASE(64, 696, 1) MTGP_CASE(64, 1727, 0) MTGP_CASE(64, 1727, 1)
     MTGP_CASE(64, 696, 2) MTGP_CASE(64, 1727, 2) MTGP_CASE(64, 696, 3) MTGP_CASE(64, 1727, 3)
 #undef MTGP_CASE
@@ -1308,10 +1323,8 @@ bool layout_supported(int bits, int cls, int layout) {
         return false;
     if (bits == 64 && cls == 3)
         return layout == 1;
-    if (layout == 2)
+    if (layout >= 2)
         return cls <= 2;
-    if (layout == 3)
-        return cls == 1 || cls == 2;
     return true;
 }
 
@@ -1319,7 +1332,7 @@ int layout_step_words(int bits, int cls, int layout) {
     if (bits == 64 && cls == 3)
         return 128;
     if (layout == 3)
-        return cls == 1 ? 512 : 1024;
+        return cls == 0 ? 256 : cls == 1 ? 512 : 1024;
     if (layout == 2)
         return cls == 0 ? 256 : 512;
     return 256;

@@ -254,8 +254,24 @@ int Context::layout_within(int lay, int mask) {
     return lay;
 }
 
-int Context::layout_for(int bits, int cls, int mask, bool one_round) const {
-    return layout_within(one_round ? layout_one_round[bits == 64][cls] : layout[bits == 64][cls], mask);
+int Context::layout_for(int bits, int cls, int mask) const {
+    return layout_within(layout[bits == 64][cls], mask);
+}
+
+int Context::layout_one_round_for(int bits, int cls, int mask, int cells, uint64_t cell, uint64_t numbers) const {
+    const int fixed = layout_one_round[bits == 64][cls];
+    if (fixed >= 0)
+        return layout_within(fixed, mask);
+    int best = 1;
+    double t = gen_ns(*this, bits, cls, 1, cells, cell, numbers);
+    for (int lay = 2; lay < kLayouts; lay++) {
+        if (!(mask >> lay & 1))
+            continue;
+        const double tl = gen_ns(*this, bits, cls, lay, cells, cell, numbers);
+        if (tl < t)
+            best = lay, t = tl;
+    }
+    return best;
 }
 
 const DevParam &Context::param(int slot) const {
@@ -892,65 +908,94 @@ void JumpBlockList::run(const Context &c, const char *d, hipStream_t s) const {
     }
 }
 
-GridModel grid_model_of(int bits, int cls, int mexp, int n) {
-    GridModel m;
-    m.jump_ns = 4.5e-5 * (double)mexp * (double)n * (double)(bits / 32) / 2;
-    m.w0 = bits == 64 ? 2.7 : 5.5;
-    m.rate = 4700;
-    // Step times of 64-set batches (2^24 + 2^24 numbers each) at 4, 8 and
-    // 12 cells per CU and of one MTGP32-11213 stream: jump launch time per
-    // jump and the generation rate's saturation in waves per CU.
-    if (bits == 32 && cls == 0)
-        m.jump_ns = 88, m.rate = 4900, m.w0 = 5.0;
-    else if (bits == 32 && cls == 1)
-        m.jump_ns = 375, m.rate = 3800;
-    else if (bits == 32 && cls == 2)
-        m.jump_ns = 880, m.rate = 3400;
-    else if (bits == 64 && cls == 0)
-        m.jump_ns = 380, m.rate = 4750;
-    else if (bits == 64 && cls == 1)
-        m.jump_ns = 1100, m.rate = 4450;
-    return m;
+double gen_ns(const Context &c, int bits, int cls, int layout, int cells, uint64_t cell, uint64_t numbers) {
+    // ns per number of a cell alone on its CU, layouts 1 to 3 (64 cells of
+    // 64 generators; the longest state a class has in the tables).
+    static constexpr double chain[2][4][3] = {
+        {{1.22, 0.85, 0.685}, {2.05, 0.715, 0.50}, {2.32, 1.135, 0.365}, {}},
+        {{2.39, 1.125, 1.025}, {2.62, 1.34, 0.595}, {3.25, 1.54, 0.73}, {2.02, 2.02, 2.02}},
+    };
+    const int lay = std::max(1, layout);
+    const int cap = std::min(c.bpc[bits == 64][cls], c.blocks_per_cu[bits == 64][cls][layout]);
+    const double rounds = std::max(1.0, (double)cells / (double)(c.cus * std::max(1, cap)));
+    // (two cells on a CU share its LDS and issue slots)
+    const double t_chain = rounds * (double)cell * chain[bits == 64][cls][lay - 1] * (cells > c.cus ? 1.1 : 1.0);
+    // GB/s of the stores alone: the fewer waves the better, and 7% less
+    // where the SIMDs do not hold 2, 4 or 8 each (64 MTGP64-23209 streams of
+    // 2^25 numbers in 1024, 1536, 2048 two-wave cells: 5475, 4747, 5136).
+    const double v = (double)cells * layout_waves(layout) / (4.0 * c.cus);
+    double even = 1, rate = v <= 2 ? 5300 : v <= 4 ? 5000 : 4900;
+    while (even < v)
+        even *= 2;
+    if (lay == 1)
+        rate = 4600;
+    else if (v > 1 && v < 0.9 * even)
+        rate *= 0.93;
+    const double t_store = (double)numbers * (bits / 8) / rate;
+    return std::pow(std::pow(t_chain, 6) + std::pow(t_store, 6), 1.0 / 6);
 }
 
-bool auto_grid(const Context &c, uint64_t total_numbers, int n_requests, int n_gens, int slots, double jump_cost,
-               const GridModel &model, uint64_t &S1, uint64_t &S2, double &frac) {
+bool auto_grid(const Context &c, uint64_t total_numbers, int n_requests, const std::vector<GridGroup> &groups, int slots,
+               double jump_cost, double cell_waves, uint64_t &S1, uint64_t &S2, double &frac) {
     const double usable = std::max(1.0, (double)slots - (double)n_requests);
     auto round256 = [](double v) { return std::max<uint64_t>(((uint64_t)v + 255) & ~255ull, 4096); };
     const double rho = jump_cost / std::max(1.0, (double)total_numbers / usable);
     if (rho > c.two_size_rho) {
-        // One round of equal cells, w per CU, w minimising the modelled step
-        // time (Context::two_size_rho).  w is a multiple of the 4 SIMDs of a
-        // CU: an uneven count leaves a CU, or a SIMD, one wave heavier, and
-        // its waves finish last (measured: MTGP64-44497 generates no faster
-        // at 5 per CU than at 4).
-        // With four-wave cells, w = 1..3 (4 to 12 waves per CU) are
-        // candidates too (MTGP64-44497: 512 four-wave cells 3.82 TB/s
-        // against 3.46 for 1024).
-        const int wmax = std::max(1, slots / std::max(1, c.cus));
-        const int wstep = model.cell_waves >= 4 ? 1 : 4;
-        double best = 0, best_t = 0;
-        for (int w = std::min(wstep, wmax); w <= wmax; w += wstep) {
-            const double jumps = std::max(0.0, (double)w * c.cus - (double)n_gens);
-            const double t_jump = c.jump_floor_ms * 1e6 + jumps * model.jump_ns;
-            const double waves = (double)w * model.cell_waves;
-            const double t_gen = model.bytes / (model.rate * (1.0 - std::exp(-waves / model.w0)));  // ns
-            const double t = t_jump + t_gen;
-            if (best == 0 || t < best_t) {
-                best = w;
-                best_t = t;
+        // One round of equal cells of the size with the least modelled step
+        // time.  Candidates: the longest stream in 1, 2, 3, ... parts (one
+        // part = no jumps at all), and 1 to 12 cells per CU over all of them
+        // (each generator's last cell is on average half full).
+        uint64_t longest = 0;
+        int gens = 0;
+        for (const GridGroup &g : groups) {
+            gens += (int)g.numbers.size();
+            for (uint64_t v : g.numbers)
+                longest = std::max(longest, v);
+        }
+        std::vector<uint64_t> sizes;
+        for (double m = 1; m <= (double)slots && (double)longest / m > 4096 / 1.2; m = std::max(m + 1, std::floor(m * 1.15)))
+            sizes.push_back(round256(std::ceil((double)longest / m)));
+        for (int w = 1; w <= std::max(1, slots / std::max(1, c.cus)); w++)
+            sizes.push_back(
+                round256(std::ceil((double)total_numbers / std::max(1.0, (double)w * c.cus - 0.5 * (double)gens))));
+        double best = -1;
+        for (uint64_t S : sizes) {
+            double t = 0, floor_ns = 0;
+            int all = 0;
+            for (const GridGroup &g : groups) {
+                uint64_t cells = 0, numbers = 0, top = 0;
+                for (uint64_t v : g.numbers) {
+                    cells += (v + S - 1) / S;
+                    numbers += v;
+                    top = std::max(top, v);
+                }
+                const int n = (int)std::min<uint64_t>(cells, INT32_MAX);
+                const double jumps = (double)cells - (double)g.numbers.size();
+                if (jumps > 0) {
+                    t += jumps * 3.6e-7 * (double)g.mexp * (double)g.mexp;
+                    floor_ns = std::max(floor_ns, 0.75 * (double)g.mexp);
+                }
+                const uint64_t cell = std::min(S, top);
+                t += gen_ns(c, g.bits, g.cls, c.layout_one_round_for(g.bits, g.cls, g.layouts, n, cell, numbers), n, cell,
+                            numbers);
+                all += n;
+            }
+            if (floor_ns > 0)
+                t += floor_ns + c.jump_floor_ms * 1e6;
+            if (all > slots && S < longest)
+                continue;
+            if (best < 0 || t < best) {
+                best = t;
+                S1 = S2 = S;
             }
         }
-        // each generator's last cell is on average half full
-        const double cells = std::max(1.0, best * (double)c.cus - 0.5 * (double)n_gens);
         frac = 0;
-        S1 = S2 = round256(std::ceil((double)total_numbers / cells));
         return true;
     }
     // Multi-round grids: rounds of slots / cell_waves cells (a large
     // MTGP64-23209 batch in two-wave cells: 4.88 TB/s at 6 per CU against
     // 4.54 at 12 and 4.55 in single-wave cells at 12).
-    const int wslots = std::max(1, (int)std::lround((double)slots / std::max(1.0, model.cell_waves_multi)));
+    const int wslots = std::max(1, (int)std::lround((double)slots / std::max(1.0, cell_waves)));
     const double wusable = std::max(1.0, (double)wslots - (double)n_requests);
     frac = c.segment_split;
     if (frac <= 0 || frac >= 1) {
@@ -1016,41 +1061,30 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
     // among the plan's generators, and the numbers-weighted mean jump cost.
     int slots = 0;
     double jcost = 0, weight = 0;
-    int active = 0;
-    GridModel model;
-    model.rate = 0;
-    model.cell_waves = 0;
-    model.cell_waves_multi = 0;
-    double w0 = 0;
+    std::vector<GridGroup> groups_of(7);
+    double cell_waves = 0;
     for (int g : named) {
         const GenRef &gr = gens[(size_t)g];
         const int b = gr.bits == 64, cls = c.class_of(gr.slot);
         const int lay = c.layout_for(gr.bits, cls, group_ok[3 * b + cls]);
-        const int lay1 = c.layout_for(gr.bits, cls, group_ok[3 * b + cls], true);
         slots = std::max(slots, c.cus * std::min(c.bpc[b][cls], c.blocks_per_cu[b][cls][lay]));
         const double nw = (double)per[(size_t)g];
         jcost += nw * jump_cost_numbers(gr.mexp, gr.n);
-        const GridModel gm = grid_model_of(gr.bits, cls, gr.mexp, gr.n);
-        model.jump_ns += nw * gm.jump_ns;
-        model.rate += nw * gm.rate;
-        model.bytes += nw * (gr.bits / 8);
-        model.cell_waves += nw * layout_waves(lay1);
-        model.cell_waves_multi += nw * layout_waves(lay);
-        w0 += nw * gm.w0;
+        cell_waves += nw * layout_waves(lay);
         weight += nw;
-        active += per[(size_t)g] > 0;
+        if (per[(size_t)g] == 0)
+            continue;
+        GridGroup &gg = groups_of[(size_t)(3 * b + cls)];
+        gg.bits = gr.bits;
+        gg.cls = cls;
+        gg.layouts = group_ok[3 * b + cls];
+        gg.mexp = std::max(gg.mexp, gr.mexp);
+        gg.numbers.push_back(per[(size_t)g]);
     }
+    groups_of.erase(std::remove_if(groups_of.begin(), groups_of.end(), [](const GridGroup &g) { return g.numbers.empty(); }),
+                    groups_of.end());
     jcost = weight > 0 ? jcost / weight : 0;
-    if (weight > 0) {
-        model.jump_ns /= weight;
-        model.rate /= weight;
-        model.w0 = w0 / weight;
-        model.cell_waves /= weight;
-        model.cell_waves_multi /= weight;
-    } else {
-        model.rate = 4700;
-        model.cell_waves = model.cell_waves_multi = 1;
-    }
+    cell_waves = weight > 0 ? cell_waves / weight : 1;
     uint64_t S1 = 0, S2 = 0;
     double frac = 0;
     // One round of cells from the step-time model: the generation launch
@@ -1062,7 +1096,7 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
     else if (opt.segment)
         S1 = S2 = opt.segment;
     else
-        one_round = auto_grid(c, all, nonempty, active, slots, jcost, model, S1, S2, frac);
+        one_round = auto_grid(c, all, nonempty, groups_of, slots, jcost, cell_waves, S1, S2, frac);
     waves_scaled = !one_round;
     one_round_grid = one_round;
     const uint64_t S = S1;
@@ -1618,9 +1652,13 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
                 L.grid = std::min(L.count, c.cus * c.jump_blocks_per_cu[L.bits == 64][L.cls]);
                 L.dyn_lds = 0;
             } else {
-                for (size_t q = i; q < j; q++)
+                uint64_t longest = 0;
+                for (size_t q = i; q < j; q++) {
                     L.numbers += cost[(size_t)order[q]];
-                L.layout = c.layout_for(L.bits, L.cls, L.layouts_ok, one_round);
+                    longest = std::max<uint64_t>(longest, cost[(size_t)order[q]]);
+                }
+                L.layout = one_round ? c.layout_one_round_for(L.bits, L.cls, L.layouts_ok, L.count, longest, L.numbers)
+                                     : c.layout_for(L.bits, L.cls, L.layouts_ok);
                 const int cap = c.blocks_per_cu[L.bits == 64][L.cls][L.layout];
                 // (the knob counts waves there; the occupancy cap counts
                 // workgroups)

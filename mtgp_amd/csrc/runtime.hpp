@@ -49,11 +49,13 @@ struct Context {
     // single-wave cells: two-wave ones measured 4.16 / 4.25 / 4.04 TB/s at 6
     // / 8 / 12 per CU against 4.21.
     int layout[2][4] = {{1, 2, 3, 1}, {2, 3, 2, 1}};
-    // The same for the step-time model's one-round grids, where MTGP32-11213
-    // also gains from two-wave cells (one stream of 2^24 + 2^24 numbers:
-    // 0.500 against 0.467 TB/s per step, generation 0.074 against 0.093 ms)
-    // while several rounds of them lose (4096 substreams: 4.21 against 4.46).
-    int layout_one_round[2][4] = {{2, 2, 3, 1}, {2, 3, 2, 1}};
+    // The same for one-round grids; -1 = the layout that the step-time model
+    // (gen_ns) has fastest for the launch's cells.  Few cells leave each CU a
+    // serial chain, which more lanes per cell shorten; many are bound by the
+    // stores, where fewer, longer waves cost less power (MTGP32-11213, 64
+    // streams of 2^23 floats, layouts 1 / 2 / 3: 512 cells 1353 / 949 / 717
+    // us, 1024 cells 697 / 506 / 451, 2048 cells 526 / 422 / 447).
+    int layout_one_round[2][4] = {{-1, -1, -1, -1}, {-1, -1, -1, -1}};
     // Resident workgroups per CU used by default.  The generation kernel is
     // held back by the board's power budget (its clock drops to 1.6-2.0 GHz
     // under full store traffic), so more waves do not generate faster but
@@ -91,18 +93,11 @@ struct Context {
     double small_rounds = 1.0;
     // Jump-cost-aware grid.  With rho = (jump cost) / (cell size of one
     // round over every slot) <= two_size_rho the two-size grid above is
-    // used; beyond it, one round of equal cells, w per CU, with w chosen to
-    // minimise the modelled step time (w a multiple of 4, the SIMDs of a CU)
-    //   jump_floor_ms + (w * CUs - generators) * t_jump
-    //     + bytes / (rate * (1 - exp(-w / w0)))
-    // with the class's measured jump time, saturated generation rate and
-    // wave scale (grid_model_of; MTGP32 waves write half the bytes per step
-    // of MTGP64 ones and need more company).  It picks the measured best of
-    // 4, 8 and 12 cells per CU for every 64-set MTGP32/MTGP64 batch (e.g.
-    // MTGP32-23209: 1.66 TB/s at 4, 2.44 at 8, 2.52 at 12) and 4 for one
-    // MTGP32-11213 stream.
+    // used; beyond it, one round of equal cells, their number minimising the
+    // modelled step time: the jumps (jump_floor_ms + 7.5e-4 us per MEXP,
+    // then 3.6e-7 ns * MEXP^2 each) and the generation launches (gen_ns).
     double two_size_rho = 0.15;
-    double jump_floor_ms = 0.15;
+    double jump_floor_ms = 0.008;
     // Two-phase launches of two-size grids (MTGP_OVERLAP=1).  Off by
     // default: on the batched MTGP32-11213 workload the side stream's jumps
     // share the generation kernel's power budget rather than hide behind its
@@ -194,7 +189,9 @@ struct Context {
     static int layout_within(int lay, int mask);
     // The default layout of (bits, class) within the mask, for a one-round
     // grid or any other.
-    int layout_for(int bits, int cls, int mask, bool one_round = false) const;
+    int layout_for(int bits, int cls, int mask) const;
+    // The layout of a one-round launch (layout_one_round).
+    int layout_one_round_for(int bits, int cls, int mask, int cells, uint64_t cell, uint64_t numbers) const;
     void sha1_of(int slot, unsigned char out[20]) const;
 };
 
@@ -232,31 +229,29 @@ uint64_t auto_segment(const Context &c, uint64_t total_numbers, int n_requests, 
 // generate).  Measured on MI355X at about 0.026 * MEXP * N numbers for
 // MTGP32-11213 and MTGP64-23209 alike.
 double jump_cost_numbers(int mexp, int n);
-// The grid model's inputs (Context::two_size_rho): for one kernel class,
-// or numbers-weighted means over the generators of a plan.
-struct GridModel {
-    double bytes = 0;     // output bytes of the plan
-    double jump_ns = 0;   // chip time of one batched jump
-    double rate = 4700;   // saturated generation rate, GB/s
-    double w0 = 5.0;      // waves per CU at which the rate is 63% of it
-    double cell_waves = 1;        // waves per cell on the one-round grid
-    double cell_waves_multi = 1;  // the same on multi-round grids
+// What the step-time model knows of one launch group of a plan: its kernel
+// class, the layouts that all its generators admit, its dearest generator's
+// MEXP, and the numbers asked of each generator.
+struct GridGroup {
+    int bits = 0, cls = 0, layouts = 0, mexp = 0;
+    std::vector<uint64_t> numbers;
 };
-// Measured on MI355X per (word size, state class); classes without a
-// measurement use jump_ns = 4.5e-5 * MEXP * N * (bits / 32) / 2 (the jump's
-// word XORs at the rate measured for MTGP32-11213 and MTGP64-23209).
-GridModel grid_model_of(int bits, int cls, int mexp, int n);
+// Modelled time of a one-round generation launch of `cells` cells, the
+// longest of `cell` numbers and `numbers` in all: one cell's serial chain,
+// the stores at the saturated rate, and their 6-norm between (within about
+// 10% of the measured times of 64 to 3072 cells in every class).
+double gen_ns(const Context &c, int bits, int cls, int layout, int cells, uint64_t cell, uint64_t numbers);
 // Cell sizes for automatic segmentation: S1 for the first `frac` of each
 // generator's positions, S2 after (frac = 0: one size).  `jump_cost` is the
 // numbers-weighted mean jump_cost_numbers of the plan's generators: when a
 // jump costs much less than a cell of one round over every slot, the
 // two-size grid (two rounds); otherwise one size, with fewer cells the
 // dearer a jump is.  `slots` counts resident workgroups; the multi-round
-// grids size their rounds in waves (slots / model.cell_waves cells), so
-// multi-wave cells keep the waves per CU of single-wave ones.  Returns true
-// for the one-round grid of the step-time model.
-bool auto_grid(const Context &c, uint64_t total_numbers, int n_requests, int n_gens, int slots, double jump_cost,
-               const GridModel &model, uint64_t &S1, uint64_t &S2, double &frac);
+// grids size their rounds in waves (slots / cell_waves cells), so multi-wave
+// cells keep the waves per CU of single-wave ones.  Returns true for the
+// one-round grid of the step-time model.
+bool auto_grid(const Context &c, uint64_t total_numbers, int n_requests, const std::vector<GridGroup> &groups, int slots,
+               double jump_cost, double cell_waves, uint64_t &S1, uint64_t &S2, double &frac);
 
 // Jump polynomials x^pos mod P kept per parameter slot for positions on a
 // grid of `cell` numbers (pos = k * cell): table T1[k] = x^(k cell) for
