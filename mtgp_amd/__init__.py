@@ -18,6 +18,7 @@ library has not been built, importing this package raises ImportError.
 """
 import ctypes as C
 import os
+import struct
 
 import numpy as np
 
@@ -522,13 +523,29 @@ class GenSet:
                "generate")
 
 
-def _requests(requests):
-    arr = (Request * max(1, len(requests)))()
-    for k, r in enumerate(requests):
-        gen, kind, count, skip, out = r
-        arr[k].gen, arr[k].kind, arr[k].count, arr[k].skip = gen, KINDS.get(kind, kind), count, skip
-        arr[k].out = out.ptr if isinstance(out, DeviceBuffer) else out
+_PACKED = "iiQQP"  # mtgp_request_t
+
+
+def _request_array(n, fields, plain=True):
+    """(Request * n) from 5 n fields in order; plain: the addresses are ints."""
+    arr = (Request * max(1, n))()
+    try:
+        if not plain:
+            raise struct.error
+        struct.pack_into(_PACKED * n, arr, 0, *fields)
+    except struct.error:  # negative or wide numbers, None: as ctypes converts them
+        for k in range(n):
+            arr[k].gen, arr[k].kind, arr[k].count, arr[k].skip, arr[k].out = fields[5 * k:5 * k + 5]
     return arr
+
+
+def _requests(requests):
+    fields, plain = [], True
+    for gen, kind, count, skip, out in requests:
+        address = out.ptr if isinstance(out, DeviceBuffer) else out
+        plain = plain and isinstance(address, int)
+        fields += (gen, KINDS.get(kind, kind), count, skip, address)
+    return _request_array(len(requests), fields, plain)
 
 
 class Plan:

@@ -895,8 +895,7 @@ void JumpBlockList::write(char *h) const {
     memcpy(h + o_folds(), folds_.data(), folds_.size() * sizeof(JumpFold));
 }
 
-void JumpBlockList::run(const Context &c, const char *d, hipStream_t s) const {
-    const JumpBlocks *g = reinterpret_cast<const JumpBlocks *>(d);
+void JumpBlockList::run(const Context &c, const char *d, const JumpBlocks *g, hipStream_t s) const {
     const JumpTile *t = reinterpret_cast<const JumpTile *>(d + o_tiles());
     const JumpShare *sh = reinterpret_cast<const JumpShare *>(d + o_shares());
     const JumpFold *f = reinterpret_cast<const JumpFold *>(d + o_folds());
@@ -1569,7 +1568,11 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
     const size_t o_jitems = align256(o_masks + mask_host.size() * 8);
     const size_t o_blists = align256(o_jitems + jitems.size() * sizeof(JumpItem));
     const size_t o_bcoef = o_blists + blocks.list_bytes();
-    const size_t work_bytes = align256(o_bcoef + bcoef_words * 4);
+    o_second = align256(o_bcoef + bcoef_words * 4);
+    const size_t second_bytes = !two_lists ? 0
+                                           : list.size() * sizeof(Item) + jitems.size() * sizeof(JumpItem) +
+                                                 blocks.groups.size() * sizeof(JumpBlocks);
+    const size_t work_bytes = align256(o_second + second_bytes);
     this->o_items = o_items;
     this->o_jitems = o_jitems;
     this->o_blists = o_blists;
@@ -1585,6 +1588,9 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
     const uint64_t dw = (uint64_t)(uintptr_t)d_work;
     d_items = reinterpret_cast<Item *>(d_work + o_items);
     d_jitems = reinterpret_cast<JumpItem *>(d_work + o_jitems);
+    d_bgroups = reinterpret_cast<JumpBlocks *>(d_work + o_blists);
+    list_states[0].clear();
+    list_states[1].clear();
     items.clear();
     item_gen.clear();
     item_io.clear();
@@ -1600,6 +1606,8 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
         item_io.push_back((uint8_t)((arena_slot[(size_t)i] ? 0 : 1) | (it.state_out ? 2 : 0)));
     }
     all_commits = commits;
+    for (size_t i = 0; two_lists && i < all_commits.size(); i++)
+        list_states[0].push_back((uint64_t)(uintptr_t)gens[(size_t)all_commits[i]].state_in);
     for (auto &ji : jitems) {
         ji.masks = dw + o_masks + ji.masks;
         ji.states_out = (uint64_t)(uintptr_t)d_jstates + ji.states_out;
@@ -1623,7 +1631,7 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
         memcpy(cf, bcopies[i].w->data(), m * 4);
         memset(cf + m, 0, (room - m) * 4);
     }
-    hip_check(hipMemcpyAsync(d_work, h_stage, work_bytes, hipMemcpyHostToDevice, opt.stream), "plan upload");
+    hip_check(hipMemcpyAsync(d_work, h_stage, o_second, hipMemcpyHostToDevice, opt.stream), "plan upload");
     if (!ev_upload)
         hip_check(hipEventCreateWithFlags(&ev_upload, hipEventDisableTiming), "hipEventCreateWithFlags");
     hip_check(hipEventRecord(ev_upload, opt.stream), "hipEventRecord");
@@ -1719,25 +1727,45 @@ void Plan::retarget(const std::vector<GenRef> &gens, hipStream_t s) {
         jitems[i].state_in = (uint64_t)(uintptr_t)gens.at((size_t)jitem_gen[i]).state_in;
     for (size_t i = 0; i < blocks.groups.size(); i++)
         blocks.groups[i].state_in = (uint64_t)(uintptr_t)gens.at((size_t)bgroup_gen[i]).state_in;
-    wait_upload();
     const size_t bb = blocks.groups.size() * sizeof(JumpBlocks);
-    if (bb) {
-        memcpy(h_stage + o_blists, blocks.groups.data(), bb);
-        hip_check(hipMemcpyAsync(d_work + o_blists, h_stage + o_blists, bb, hipMemcpyHostToDevice, s), "plan upload");
-    }
     const size_t ib = items.size() * sizeof(Item), jb = jitems.size() * sizeof(JumpItem);
-    if (ib) {
-        memcpy(h_stage + o_items, items.data(), ib);
-        hip_check(hipMemcpyAsync(d_work + o_items, h_stage + o_items, ib, hipMemcpyHostToDevice, s), "plan upload");
+    size_t at_items = o_items, at_jitems = o_jitems, at_groups = o_blists;
+    commits = all_commits;
+    if (two_lists) {
+        std::vector<uint64_t> states;
+        for (int g : all_commits)
+            states.push_back((uint64_t)(uintptr_t)gens.at((size_t)g).state_in);
+        const bool known = states == list_states[0] || states == list_states[1];
+        // (an unknown pair of slots replaces the list that is not in use)
+        const int which = known ? states != list_states[0] : d_items == reinterpret_cast<Item *>(d_work + o_items);
+        if (which) {
+            at_items = o_second;
+            at_jitems = at_items + ib;
+            at_groups = at_jitems + jb;
+        }
+        d_items = reinterpret_cast<Item *>(d_work + at_items);
+        d_jitems = reinterpret_cast<JumpItem *>(d_work + at_jitems);
+        d_bgroups = reinterpret_cast<JumpBlocks *>(d_work + at_groups);
+        if (known)
+            return;
+        list_states[which].clear();
     }
-    if (jb) {
-        memcpy(h_stage + o_jitems, jitems.data(), jb);
-        hip_check(hipMemcpyAsync(d_work + o_jitems, h_stage + o_jitems, jb, hipMemcpyHostToDevice, s), "plan upload");
-    }
+    wait_upload();
+    const auto upload = [&](size_t at, const void *src, size_t bytes) {
+        if (!bytes)
+            return;
+        memcpy(h_stage + at, src, bytes);
+        hip_check(hipMemcpyAsync(d_work + at, h_stage + at, bytes, hipMemcpyHostToDevice, s), "plan upload");
+    };
+    upload(at_groups, blocks.groups.data(), bb);
+    upload(at_items, items.data(), ib);
+    upload(at_jitems, jitems.data(), jb);
+    if (two_lists)
+        for (int g : all_commits)
+            list_states[at_items != o_items].push_back((uint64_t)(uintptr_t)gens.at((size_t)g).state_in);
     if (!ev_upload)
         hip_check(hipEventCreateWithFlags(&ev_upload, hipEventDisableTiming), "hipEventCreateWithFlags");
     hip_check(hipEventRecord(ev_upload, s), "hipEventRecord");
-    commits = all_commits;
 }
 
 void Plan::reserve(size_t work_bytes, size_t jstates_bytes) {
@@ -1787,7 +1815,7 @@ void Plan::run_launches(int part, int phase, hipStream_t s) {
     const size_t iq = merged ? 2 * (launches.size() + jlaunches.size()) : 0;
     const size_t jq = iq + 2 * I.size();
     if (part == 0 && phase <= 0)  // (blocked jumps of both phases run with phase 0)
-        blocks.run(*ctx, d_work + o_blists, s);
+        blocks.run(*ctx, d_work + o_blists, d_bgroups, s);
     for (size_t k = 0; part == 0 && k < J.size(); k++) {
         const Launch &L = J[k];
         if (!merged && L.phase != phase)
@@ -2046,7 +2074,7 @@ static bool device_jump_blocks(Context &c, int slot, int bits, int mexp, const v
         memcpy(h + o_in, in, wbytes);
     hip_check(hipMemcpyAsync(d, h, host_io ? o_in + wbytes : o_in, hipMemcpyHostToDevice, nullptr),
               "hipMemcpyAsync jump workspace");
-    L.run(c, d, nullptr);
+    L.run(c, d, reinterpret_cast<const JumpBlocks *>(d), nullptr);
     if (host_io)
         hip_check(hipMemcpyAsync(h + o_out, d + o_out, wbytes, hipMemcpyDeviceToHost, nullptr),
                   "hipMemcpyAsync jumped window");
@@ -2871,8 +2899,10 @@ int mtgp_genset_generate(mtgp_genset_t *s, const mtgp_request_t *reqs, int nreq,
     std::lock_guard<std::mutex> lk(s->gen_mu);
     if (nreq < 0 || (nreq > 0 && !reqs))
         throw Error("bad request list");
-    if (!s->gen_plan)
+    if (!s->gen_plan) {
         s->gen_plan = std::make_unique<Plan>();
+        s->gen_plan->two_lists = true;
+    }
     Plan &plan = *s->gen_plan;
     std::vector<mtgp_request_t> rv(reqs, reqs + nreq);
     uint64_t epoch;
@@ -2899,8 +2929,13 @@ int mtgp_genset_generate(mtgp_genset_t *s, const mtgp_request_t *reqs, int nreq,
         s->gen_reqs = rv;
         s->gen_epoch = epoch;
     }
-    plan.launch((hipStream_t)stream);
-    hip_check(hipStreamSynchronize((hipStream_t)stream), "hipStreamSynchronize");
+    try {
+        plan.launch((hipStream_t)stream);
+        hip_check(hipStreamSynchronize((hipStream_t)stream), "hipStreamSynchronize");
+    } catch (...) {
+        s->gen_reqs.clear();  // (its lists may not have arrived)
+        throw;
+    }
     for (int g : plan.commits)
         s->set_cur(g, s->cur[(size_t)g] ^ 1);
     return 0;
@@ -3038,7 +3073,7 @@ int mtgp_genset_substreams(mtgp_genset_t *s, const void *base, const char *hex) 
         grow_pinned(c.jump_h, c.jump_hcap, wbytes);
         memcpy(c.jump_h, base, wbytes);
         hip_check(hipMemcpyAsync(s->state(0, 0), c.jump_h, wbytes, hipMemcpyHostToDevice, nullptr), "hipMemcpyAsync base");
-        W.blocks.run(c, W.d + W.o_lists, nullptr);
+        W.blocks.run(c, W.d + W.o_lists, reinterpret_cast<const JumpBlocks *>(W.d + W.o_lists), nullptr);
         hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");
         for (int g = 0; g < G; g++)
             s->set_cur(g, 0);

@@ -329,8 +329,8 @@ class JumpBlockList {
     // The device lists: their size, and their bytes to an upload buffer.
     size_t list_bytes() const;
     void write(char *h) const;
-    // Every launch, from the lists at d_lists.
-    void run(const Context &c, const char *d_lists, hipStream_t s) const;
+    // Every launch, from the lists at d_lists and the groups at d_groups.
+    void run(const Context &c, const char *d_lists, const JumpBlocks *d_groups, hipStream_t s) const;
     int launches() const { return 2 * (int)launches_.size(); }
     std::vector<JumpBlocks> groups;
 
@@ -406,6 +406,16 @@ struct Plan {
     JumpBlockList blocks;
     std::vector<int32_t> bgroup_gen;
     size_t o_blists = 0;
+    // Work lists for both state slots (set before build by an owner that
+    // waits for each launch and never captures one): what a retarget changes
+    // is kept twice, at the build's place and at o_second, and a call whose
+    // generators' slots are those of one of the two uploads nothing.  Without
+    // it every retarget overwrites the build's place, which a captured graph
+    // reads.  (One stream of 10^6 floats: 42 us a call against 50; of 2^24 words 78 against 101.)
+    bool two_lists = false;
+    size_t o_second = 0;
+    std::vector<uint64_t> list_states[2];  // the committed generators' state_in of each; empty = unwritten
+    JumpBlocks *d_bgroups = nullptr;
     hipEvent_t ev_upload = nullptr;    // the last upload from h_stage
     // Device copies: one grow-only workspace [items | segs | polys | masks |
     // jump items], the jumped-state arena and the work-queue counters.

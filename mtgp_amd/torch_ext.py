@@ -16,6 +16,7 @@ is mapped and fails otherwise.
     gs.generate_([(0, mt.KIND_CLOSE_OPEN, x), (1, mt.KIND_CLOSE_OPEN, y)])
 """
 import ctypes as C
+import functools
 import os
 
 import torch
@@ -49,6 +50,7 @@ _UINT32 = getattr(torch, "uint32", torch.int32)
 _UINT64 = getattr(torch, "uint64", torch.int64)
 
 
+@functools.lru_cache(maxsize=64)
 def _dtypes(bits, kind):
     ints = (_UINT32, torch.int32) if bits == 32 else (_UINT64, torch.int64)
     floats = (torch.float32,) if bits == 32 else (torch.float64,)
@@ -67,19 +69,19 @@ class TensorGenSet(M.GenSet):
         tensor (contiguous, on the GPU, of the kind's element type) is
         filled completely, in order, on `stream` (default: torch's current
         stream), which is synchronised before returning."""
-        reqs = []
+        fields, n, specs = [], 0, self.specs
         for r in requests:
             gen, kind, t = r[0], r[1], r[2]
-            skip = r[3] if len(r) > 3 else 0
-            bits = self.specs[gen][0]
+            bits = specs[gen][0]
             if not t.is_cuda or not t.is_contiguous():
                 raise ValueError("tensor must be contiguous and on the GPU")
             if t.dtype not in _dtypes(bits, kind):
                 raise TypeError("tensor dtype %s does not hold kind %d of an MTGP%d generator" % (t.dtype, kind, bits))
-            reqs.append((gen, kind, t.numel(), skip, t.data_ptr()))
+            fields += (gen, M.KINDS.get(kind, kind), t.numel(), r[3] if len(r) > 3 else 0, t.data_ptr())
+            n += 1
         s = stream if stream is not None else torch.cuda.current_stream()
-        arr = M._requests(reqs)
-        M._check(M._lib.mtgp_genset_generate(self.h, arr, len(reqs), C.c_void_p(s.cuda_stream)), "generate")
+        arr = M._request_array(n, fields)
+        M._check(M._lib.mtgp_genset_generate(self.h, arr, n, C.c_void_p(s.cuda_stream)), "generate")
 
 
 class Generator:
