@@ -1233,11 +1233,9 @@ struct KernelOf;
 // steps of two words per lane for the N <= 726/696 classes).
 template <int NMAX, int LAYOUT>
 struct KernelOf<32, NMAX, LAYOUT, 4> {
-    static constexpr int waves = LAYOUT == 3 ? 4 : LAYOUT == 2 ? 2 : 1;
+    static constexpr int waves = LAYOUT == 3 ? (NMAX <= 726 ? 4 : 8) : LAYOUT == 2 ? 2 : 1;
     static constexpr int step_layout = LAYOUT >= 2 ? 1 : LAYOUT;
-    static constexpr int wpl = LAYOUT == 3 && NMAX <= 351                                  ? 1
-                               : (LAYOUT == 2 && NMAX <= 351) || (LAYOUT == 3 && NMAX <= 726) ? 2
-                                                                                              : 4;
+    static constexpr int wpl = LAYOUT == 3 ? (NMAX <= 351 ? 1 : 2) : LAYOUT == 2 && NMAX <= 351 ? 2 : 4;
     static constexpr int k = wpl == 1 ? kKLatency : kK;
     static constexpr auto fn = mtgp32_items_kernel<NMAX, k, step_layout, waves, wpl>;
     static std::string name() {
@@ -1247,11 +1245,9 @@ struct KernelOf<32, NMAX, LAYOUT, 4> {
 };
 template <int NMAX, int LAYOUT, int WPL>
 struct KernelOf<64, NMAX, LAYOUT, WPL> {
-    static constexpr int waves = LAYOUT == 3 ? 4 : LAYOUT == 2 ? 2 : 1;
+    static constexpr int waves = LAYOUT == 3 ? (NMAX <= 726 ? 4 : 8) : LAYOUT == 2 ? 2 : 1;
     static constexpr int step_layout = LAYOUT >= 2 ? 1 : LAYOUT;
-    static constexpr int wpl = LAYOUT == 3 && NMAX <= 363                                  ? 1
-                               : (LAYOUT == 2 && NMAX <= 363) || (LAYOUT == 3 && NMAX <= 696) ? 2
-                                                                                              : WPL;
+    static constexpr int wpl = LAYOUT == 3 ? (NMAX <= 363 ? 1 : 2) : LAYOUT == 2 && NMAX <= 363 ? 2 : WPL;
     static constexpr int k = wpl == 1 ? kKLatency : kK;
     static constexpr auto fn = mtgp64_items_kernel<NMAX, k, step_layout, wpl, waves>;
     static std::string name() {

@@ -911,14 +911,17 @@ double gen_ns(const Context &c, int bits, int cls, int layout, int cells, uint64
     // ns per number of a cell alone on its CU, layouts 1 to 3 (64 cells of
     // 64 generators; the longest state a class has in the tables).
     static constexpr double chain[2][4][3] = {
-        {{1.22, 0.85, 0.685}, {2.05, 0.715, 0.50}, {2.32, 1.135, 0.365}, {}},
-        {{2.39, 1.125, 1.025}, {2.62, 1.34, 0.595}, {3.25, 1.54, 0.73}, {2.02, 2.02, 2.02}},
+        {{1.22, 0.85, 0.685}, {2.05, 0.715, 0.50}, {2.32, 1.135, 0.29}, {}},
+        {{2.39, 1.125, 1.025}, {2.62, 1.34, 0.595}, {3.25, 1.54, 0.405}, {2.02, 2.02, 2.02}},
     };
     const int lay = std::max(1, layout);
     const int cap = std::min(c.bpc[bits == 64][cls], c.blocks_per_cu[bits == 64][cls][layout]);
     const double rounds = std::max(1.0, (double)cells / (double)(c.cus * std::max(1, cap)));
-    // (two cells on a CU share its LDS and issue slots)
-    const double t_chain = rounds * (double)cell * chain[bits == 64][cls][lay - 1] * (cells > c.cus ? 1.1 : 1.0);
+    // (cells on one CU share its LDS and issue slots: 64 MTGP32-44497 streams
+    // in 256, 320, 384 cells 687, 685, 604 us)
+    static constexpr double shared[4] = {1.05, 1.15, 1.25, 1.05};
+    const double t_chain =
+        rounds * (double)cell * chain[bits == 64][cls][lay - 1] * (cells > c.cus ? shared[cls] : 1.0);
     // GB/s of the stores alone: the fewer waves the better, and 7% less
     // where the SIMDs do not hold 2, 4 or 8 each (64 MTGP64-23209 streams of
     // 2^25 numbers in 1024, 1536, 2048 two-wave cells: 5475, 4747, 5136).
@@ -971,7 +974,7 @@ bool auto_grid(const Context &c, uint64_t total_numbers, int n_requests, const s
                 const int n = (int)std::min<uint64_t>(cells, INT32_MAX);
                 const double jumps = (double)cells - (double)g.numbers.size();
                 if (jumps > 0) {
-                    t += jumps * 3.6e-7 * (double)g.mexp * (double)g.mexp;
+                    t += jumps * (3.1e-7 * (double)g.mexp + 6e-4) * (double)g.mexp;
                     floor_ns = std::max(floor_ns, 0.75 * (double)g.mexp);
                 }
                 const uint64_t cell = std::min(S, top);

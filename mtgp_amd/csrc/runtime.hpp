@@ -95,7 +95,7 @@ struct Context {
     // round over every slot) <= two_size_rho the two-size grid above is
     // used; beyond it, one round of equal cells, their number minimising the
     // modelled step time: the jumps (jump_floor_ms + 7.5e-4 us per MEXP,
-    // then 3.6e-7 ns * MEXP^2 each) and the generation launches (gen_ns).
+    // then 3.1e-7 ns * MEXP^2 + 6e-4 ns * MEXP each) and the generation launches (gen_ns).
     double two_size_rho = 0.15;
     double jump_floor_ms = 0.008;
     // Two-phase launches of two-size grids (MTGP_OVERLAP=1).  Off by
