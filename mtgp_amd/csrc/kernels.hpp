@@ -27,8 +27,8 @@ constexpr int kLayouts = 4;
 // Whether (bits, cls) has a kernel of that layout, and its words per step.
 bool layout_supported(int bits, int cls, int layout);
 int layout_step_words(int bits, int cls, int layout);
-// What a cell of a layout takes of the workgroups-per-CU knob: its waves (four
-// also for the eight of layout 3's class 2, which three per CU suit best).
+// Waves per cell of a layout, for the model's waves per SIMD (layout 3's class
+// 2 has eight, and fills a CU as four do).
 inline int layout_waves(int layout) { return layout == 3 ? 4 : layout == 2 ? 2 : 1; }
 // Kernel entry (for occupancy queries) and its workgroup size.
 const void *kernel_fn(int bits, int cls, int layout);

@@ -255,7 +255,19 @@ int Context::layout_within(int lay, int mask) {
 }
 
 int Context::layout_for(int bits, int cls, int mask) const {
-    return layout_within(layout[bits == 64][cls], mask);
+    const int fixed = layout[bits == 64][cls];
+    return layout_within(fixed >= 0 ? fixed : kLayouts - 1, mask);
+}
+
+int Context::per_cu(int bits, int cls, int layout, int cells, int knob) const {
+    const int cap = blocks_per_cu[bits == 64][cls][layout];
+    const int b = std::min(knob, cap);
+    // Up to half a round more cells than slots (e.g. one cell per generator
+    // for thousands of generators) run as one round when the occupancy limit
+    // allows: a partial second round would leave most waves idle.
+    if (cells > cus * b && cells <= cus * cap && 2 * cells <= 3 * cus * b)
+        return (cells + cus - 1) / cus;
+    return b;
 }
 
 int Context::layout_one_round_for(int bits, int cls, int mask, int cells, uint64_t cell, uint64_t numbers) const {
@@ -915,8 +927,8 @@ double gen_ns(const Context &c, int bits, int cls, int layout, int cells, uint64
         {{2.39, 1.125, 1.025}, {2.62, 1.34, 0.595}, {3.25, 1.54, 0.405}, {2.02, 2.02, 2.02}},
     };
     const int lay = std::max(1, layout);
-    const int cap = std::min(c.bpc[bits == 64][cls], c.blocks_per_cu[bits == 64][cls][layout]);
-    const double rounds = std::max(1.0, (double)cells / (double)(c.cus * std::max(1, cap)));
+    const int per = c.per_cu(bits, cls, layout, cells, c.bpc[bits == 64][cls]);
+    const double rounds = std::max(1.0, (double)cells / (double)(c.cus * std::max(1, per)));
     // (cells on one CU share its LDS and issue slots: 64 MTGP32-44497 streams
     // in 256, 320, 384 cells 687, 685, 604 us)
     static constexpr double shared[4] = {1.05, 1.15, 1.25, 1.05};
@@ -933,8 +945,11 @@ double gen_ns(const Context &c, int bits, int cls, int layout, int cells, uint64
         rate = 4600;
     else if (v > 1 && v < 0.9 * even)
         rate *= 0.93;
+    if (rounds > 1)
+        rate = lay == 1 ? 4700 : lay == 2 ? 4950 : 5100;
     const double t_store = (double)numbers * (bits / 8) / rate;
-    return std::pow(std::pow(t_chain, 6) + std::pow(t_store, 6), 1.0 / 6);
+    const double t = std::pow(std::pow(t_chain, 6) + std::pow(t_store, 6), 1.0 / 6);
+    return rounds > 1 ? std::hypot(t, 10.0 * cells) : t;
 }
 
 bool auto_grid(const Context &c, uint64_t total_numbers, int n_requests, const std::vector<GridGroup> &groups, int slots,
@@ -1068,7 +1083,7 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
     for (int g : named) {
         const GenRef &gr = gens[(size_t)g];
         const int b = gr.bits == 64, cls = c.class_of(gr.slot);
-        const int lay = c.layout_for(gr.bits, cls, group_ok[3 * b + cls]);
+        const int lay = Context::layout_within(Context::sizing[b][cls], group_ok[3 * b + cls]);
         slots = std::max(slots, c.cus * std::min(c.bpc[b][cls], c.blocks_per_cu[b][cls][lay]));
         const double nw = (double)per[(size_t)g];
         jcost += nw * jump_cost_numbers(gr.mexp, gr.n);
@@ -1678,16 +1693,18 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
                     one_round ||
                     (opt.cache && L.count <= c.cus * std::min(knob, c.blocks_per_cu[L.bits == 64][L.cls][model]));
                 L.layout = fits ? model : c.layout_for(L.bits, L.cls, L.layouts_ok);
-                const int cap = c.blocks_per_cu[L.bits == 64][L.cls][L.layout];
-                // (on multi-round grids the knob counts waves; the occupancy
-                // cap counts workgroups)
-                int bpc = std::min(fits ? knob : std::max(1, knob / layout_waves(L.layout)), cap);
-                // Up to half a round more cells than slots (e.g. one cell per
-                // generator for thousands of generators) run as one round
-                // when the occupancy limit allows: a partial second round
-                // would leave most waves idle.
-                if (L.count > c.cus * bpc && L.count <= c.cus * cap && 2 * L.count <= 3 * c.cus * bpc)
-                    bpc = (L.count + c.cus - 1) / c.cus;
+                // Cells that layout 1 holds in one round and that are too
+                // short to hide the claims stay there (4096 MTGP32-11213
+                // cells of 2^12, 2^14, 2^16 words: 21, 54, 233 us against 55,
+                // 76, 220).
+                if (!fits && c.layout[L.bits == 64][L.cls] < 0 &&
+                    L.count <= c.cus * c.per_cu(L.bits, L.cls, 1, L.count, knob) &&
+                    gen_ns(c, L.bits, L.cls, 1, L.count, longest, L.numbers) <
+                        gen_ns(c, L.bits, L.cls, L.layout, L.count, longest, L.numbers))
+                    L.layout = 1;
+                const int bpc = c.per_cu(
+                    L.bits, L.cls, L.layout, L.count,
+                    fits ? knob : c.rounds_knob(L.bits, L.cls, L.layout, L.count));
                 L.grid = std::min(L.count, c.cus * bpc);
                 L.dyn_lds = c.lds_reserve(kernel_fn(L.bits, L.cls, L.layout), kernel_threads(L.bits, L.cls, L.layout), bpc);
             }
@@ -1874,7 +1891,7 @@ void Plan::configure(int layout, int bpc) {
         }
         int cap = ctx->blocks_per_cu[L.bits == 64][L.cls][L.layout];
         cap = std::min(cap, bpc > 0 ? bpc
-                                    : waves_scaled ? std::max(1, ctx->bpc[L.bits == 64][L.cls] / layout_waves(L.layout))
+                                    : waves_scaled ? ctx->rounds_knob(L.bits, L.cls, L.layout, L.count)
                                                    : ctx->bpc[L.bits == 64][L.cls]);
         L.grid = std::min(L.count, ctx->cus * cap);
         L.dyn_lds = ctx->lds_reserve(kernel_fn(L.bits, L.cls, L.layout), kernel_threads(L.bits, L.cls, L.layout), cap);

@@ -39,16 +39,28 @@ struct Context {
     // (class 3 exists for 64-bit only; kernels.hpp).
     int blocks_per_cu[2][4][4] = {};  // [bits == 64][class][layout]
     int jump_blocks_per_cu[2][4] = {};
-    // Multi-wave cells by default where they measured faster: on 64-set
-    // batches of MTGP32-23209 / MTGP64-23209, two-wave cells (layout 2) 3.32
-    // / 4.09 TB/s per step against 2.60 / 3.86-3.95 with single-wave cells;
-    // MTGP32-44497 / MTGP64-44497, four-wave cells (layout 3) on 768 / 512
-    // cells 3.03 / 3.76 against 2.22 / 3.49 with two-wave cells and 1.78 /
-    // 2.83 with single-wave ones (more waves per CU from fewer cells, so
-    // fewer start-state jumps).  Batched MTGP32-11213 keeps
-    // single-wave cells: two-wave ones measured 4.16 / 4.25 / 4.04 TB/s at 6
-    // / 8 / 12 per CU against 4.21.
-    int layout[2][4] = {{1, 2, 3, 1}, {2, 3, 2, 1}};
+    // The layout of launches of several rounds; -1 = layout 3 where the set
+    // has it.  The stores are what bounds those, and fewer, faster streams
+    // write faster: 4096 MTGP32-11213 cells of 2^20 words in layout 1 (16 per
+    // CU) 3490 us, 2 (6, 8) 3503, 3499, 3 (6, 8) 3384, 3314; 10000 of 2^17
+    // 1029, 1029, 971, 967, 985; 4096 MTGP32-23209 cells of 2^20 in layouts 2
+    // and 3 (6) 3329, 3226; MTGP64-44497 of 2^18 in layout 3 (3, 6) 1501, 1573.
+    int layout[2][4] = {{-1, -1, -1, -1}, {-1, -1, -1, -1}};
+    // Workgroups per CU of such a launch of `cells` cells (at most the
+    // occupancy limit): the knob (bpc) halved or quartered, but whole where
+    // layout 3 then has two rounds at most (6 and 8 per CU: 3072 and 4096
+    // MTGP32-11213 cells of 17 GB 3576, 3384 and 3352, 3314 us; 6000, 8192
+    // 3155, 3126 and 3246, 3158; 4096 of MTGP32-23209 3226 and 3139).
+    int rounds_knob(int bits, int cls, int layout, int cells) const {
+        const int knob = bpc[bits == 64][cls], share = layout == 3 ? (bits == 64 && cls == 1 ? 4 : 2) : layout == 2 ? 2 : 1;
+        const int cap = std::min(knob, blocks_per_cu[bits == 64][cls][layout]);
+        return layout == 3 && share == 2 && cells <= 2 * cus * cap ? cap : std::max(1, knob / share);
+    }
+    // The layout whose occupancy and waves size the cells of such grids: more
+    // cells would cost more jumps than the even finish gains (the two-size
+    // grid of the batched MTGP32-11213 workload for 6, 8 and 12 cells per CU
+    // in a round: 3.86, 3.83, 3.77 ms).
+    static constexpr int sizing[2][4] = {{1, 2, 3, 1}, {2, 3, 2, 1}};
     // The same for one-round grids; -1 = the layout that the step-time model
     // (gen_ns) has fastest for the launch's cells.  Few cells leave each CU a
     // serial chain, which more lanes per cell shorten; many are bound by the
@@ -56,7 +68,8 @@ struct Context {
     // streams of 2^23 floats, layouts 1 / 2 / 3: 512 cells 1353 / 949 / 717
     // us, 1024 cells 697 / 506 / 451, 2048 cells 526 / 422 / 447).
     int layout_one_round[2][4] = {{-1, -1, -1, -1}, {-1, -1, -1, -1}};
-    // Resident workgroups per CU used by default.  The generation kernel is
+    // Resident workgroups per CU used by default, counted in single waves on
+    // several rounds (rounds_knob).  The generation kernel is
     // held back by the board's power budget (its clock drops to 1.6-2.0 GHz
     // under full store traffic), so more waves do not generate faster but
     // do mean more cells, hence more jumps: on the batched MTGP32-11213
@@ -190,6 +203,9 @@ struct Context {
     // The default layout of (bits, class) within the mask, for a one-round
     // grid or any other.
     int layout_for(int bits, int cls, int mask) const;
+    // Workgroups per CU for `cells` cells, `knob` at most unless the cells
+    // are up to half a round more and the occupancy limit allows them.
+    int per_cu(int bits, int cls, int layout, int cells, int knob) const;
     // The layout of a one-round launch (layout_one_round).
     int layout_one_round_for(int bits, int cls, int mask, int cells, uint64_t cell, uint64_t numbers) const;
     void sha1_of(int slot, unsigned char out[20]) const;
@@ -236,10 +252,11 @@ struct GridGroup {
     int bits = 0, cls = 0, layouts = 0, mexp = 0;
     std::vector<uint64_t> numbers;
 };
-// Modelled time of a one-round generation launch of `cells` cells, the
-// longest of `cell` numbers and `numbers` in all: one cell's serial chain,
-// the stores at the saturated rate, and their 6-norm between (within about
-// 10% of the measured times of 64 to 3072 cells in every class).
+// Modelled time of a generation launch of `cells` cells, the longest of `cell`
+// numbers and `numbers` in all: one cell's serial chain, the stores at the
+// saturated rate, and their 6-norm between (within about 10% of the measured
+// times of 64 to 3072 cells in every class).  Beyond one round every cell is
+// claimed, 10 ns each on one counter.
 double gen_ns(const Context &c, int bits, int cls, int layout, int cells, uint64_t cell, uint64_t numbers);
 // Cell sizes for automatic segmentation: S1 for the first `frac` of each
 // generator's positions, S2 after (frac = 0: one size).  `jump_cost` is the
@@ -247,8 +264,7 @@ double gen_ns(const Context &c, int bits, int cls, int layout, int cells, uint64
 // jump costs much less than a cell of one round over every slot, the
 // two-size grid (two rounds); otherwise one size, with fewer cells the
 // dearer a jump is.  `slots` counts resident workgroups; the multi-round
-// grids size their rounds in waves (slots / cell_waves cells), so multi-wave
-// cells keep the waves per CU of single-wave ones.  Returns true for the
+// grids size their rounds in waves (slots / cell_waves cells).  Returns true for the
 // one-round grid of the step-time model.
 bool auto_grid(const Context &c, uint64_t total_numbers, int n_requests, const std::vector<GridGroup> &groups, int slots,
                double jump_cost, double cell_waves, uint64_t &S1, uint64_t &S2, double &frac);
