@@ -929,11 +929,17 @@ double gen_ns(const Context &c, int bits, int cls, int layout, int cells, uint64
     const int lay = std::max(1, layout);
     const int per = c.per_cu(bits, cls, layout, cells, c.bpc[bits == 64][cls]);
     const double rounds = std::max(1.0, (double)cells / (double)(c.cus * std::max(1, per)));
+    // The longest cells run first; a second round that is nearly empty still
+    // takes as long as one of the shortest cells (2112 equal MTGP32-11213
+    // cells on 2048 slots 983 us, 1856 976; 2286 1050, 1989 971).
+    const double shortest = std::max(0.0, 2.0 * (double)numbers / std::max(1, cells) - (double)cell);
+    const double serial =
+        std::max((double)cell + (std::ceil(rounds) - 1) * shortest, rounds * (double)numbers / std::max(1, cells));
     // (cells on one CU share its LDS and issue slots: 64 MTGP32-44497 streams
     // in 256, 320, 384 cells 687, 685, 604 us)
     static constexpr double shared[4] = {1.05, 1.15, 1.25, 1.05};
     const double t_chain =
-        rounds * (double)cell * chain[bits == 64][cls][lay - 1] * (cells > c.cus ? shared[cls] : 1.0);
+        serial * chain[bits == 64][cls][lay - 1] * (cells > c.cus ? shared[cls] : 1.0);
     // GB/s of the stores alone: the fewer waves the better, and 7% less
     // where the SIMDs do not hold 2, 4 or 8 each (64 MTGP64-23209 streams of
     // 2^25 numbers in 1024, 1536, 2048 two-wave cells: 5475, 4747, 5136).
