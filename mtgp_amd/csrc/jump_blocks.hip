@@ -376,7 +376,13 @@ __global__ __launch_bounds__(kTileThreads, 2) void jump_tiles_kernel(const JumpB
 }
 
 // ------------------------------------------------------------------- folds
-// One workgroup per JumpFold: T threads, S numbers per step.
+// One workgroup per JumpFold: T threads, S numbers per step.  The chain of a
+// block is 1 to 4 steps, no longer than a load of its part can take (the
+// tiles wrote it from any XCD, so it misses the L2), so parts are loaded
+// kFoldAhead blocks ahead (one and four ahead, one jump: MTGP32-11213 8.8 and
+// 7.6 us, MTGP64-23209 19.8 and 16.9, MTGP64-44497 28.5 and 24.4, MTGP64-
+// 110503 70 and 60).
+constexpr int kFoldAhead = 4;
 template <int BITS, int NMAX, int S, int T>
 __global__ __launch_bounds__(T) void jump_folds_kernel(const JumpBlocks *__restrict__ groups,
                                                        const JumpFold *__restrict__ folds,
@@ -391,52 +397,61 @@ __global__ __launch_bounds__(T) void jump_folds_kernel(const JumpBlocks *__restr
     const DevParam &D = params[G.param];
     const Rec p = rec_of(D);
     const int pw = (p.n + kJbGroup - 1) / kJbGroup * kJbGroup;
-    const gu32 *P = reinterpret_cast<const gu32 *>(G.parts) + ((uint64_t)(I.b + 1) * (uint64_t)G.ch - 1) * (uint64_t)(PL * pw);
+    const gu32 *P = reinterpret_cast<const gu32 *>(G.parts) + (uint64_t)I.b * (uint64_t)G.ch * (uint64_t)(PL * pw);
     if (t < 16)
         tbl[t] = D.tbl[t];
-    uint32_t part[PL][NJ];
+    // (lanes beyond the window repeat its last word)
+    int at[NJ];
 #pragma unroll
     for (int m = 0; m < NJ; m++)
-#pragma unroll
-        for (int h = 0; h < PL; h++)
-            part[h][m] = t + T * m < p.n ? P[h * pw + t + T * m] : 0u;
-    for (int a = G.ch - 1;; a--) {
-#pragma unroll
-        for (int m = 0; m < NJ; m++)
-#pragma unroll
-            for (int h = 0; h < PL; h++)
-                if (t + T * m < p.n)
-                    buf[h][t + T * m] = part[h][m];
-        if (a == 0)
-            break;
-        P -= PL * pw;
+        at[m] = t + T * m < p.n ? t + T * m : p.n - 1;
+    uint32_t part[PL][NJ], ring[kFoldAhead][PL][NJ];
+    const auto load = [&](uint32_t(&r)[PL][NJ], int a) {
+        const gu32 *q = P + (uint64_t)(a > 0 ? a : 0) * (uint64_t)(PL * pw);
 #pragma unroll
         for (int m = 0; m < NJ; m++)
 #pragma unroll
             for (int h = 0; h < PL; h++)
-                part[h][m] = t + T * m < p.n ? P[h * pw + t + T * m] : 0u;
-        __syncthreads();
-        for (int k = 0; k < kJbBlock; k += S) {
-            uint32_t rh[S / T], rl[S / T];
+                r[h][m] = q[h * pw + at[m]];
+    };
+    load(part, G.ch - 1);
 #pragma unroll
-            for (int i = 0; i < S / T; i++)
-                next_word<BITS>(p, tbl, buf[0], buf[PL - 1], k + t + T * i, rh[i], rl[i]);
+    for (int i = 0; i < kFoldAhead; i++)
+        load(ring[i], G.ch - 2 - i);
+    for (int a = G.ch - 2; a >= 0;) {
 #pragma unroll
-            for (int i = 0; i < S / T; i++) {
-                buf[0][p.n + k + t + T * i] = rh[i];
-                if (BITS == 64)
-                    buf[PL - 1][p.n + k + t + T * i] = rl[i];
+        for (int i = 0; i < kFoldAhead; i++) {
+            if (a < 0)
+                break;
+#pragma unroll
+            for (int m = 0; m < NJ; m++)
+#pragma unroll
+                for (int h = 0; h < PL; h++)
+                    buf[h][at[m]] = part[h][m];
+            __syncthreads();
+            for (int k = 0; k < kJbBlock; k += S) {
+                uint32_t rh[S / T], rl[S / T];
+#pragma unroll
+                for (int i2 = 0; i2 < S / T; i2++)
+                    next_word<BITS>(p, tbl, buf[0], buf[PL - 1], k + t + T * i2, rh[i2], rl[i2]);
+#pragma unroll
+                for (int i2 = 0; i2 < S / T; i2++) {
+                    buf[0][p.n + k + t + T * i2] = rh[i2];
+                    if (BITS == 64)
+                        buf[PL - 1][p.n + k + t + T * i2] = rl[i2];
+                }
+                __syncthreads();
             }
-            __syncthreads();
+#pragma unroll
+            for (int m = 0; m < NJ; m++)
+#pragma unroll
+                for (int h = 0; h < PL; h++)
+                    part[h][m] = ring[i][h][m] ^ buf[h][kJbBlock + at[m]];
+            load(ring[i], a - kFoldAhead);
+            a--;
+            if (NMAX > kJbBlock)  // the window's old and new places overlap
+                __syncthreads();
         }
-#pragma unroll
-        for (int m = 0; m < NJ; m++)
-#pragma unroll
-            for (int h = 0; h < PL; h++)
-                if (t + T * m < p.n)
-                    part[h][m] ^= buf[h][kJbBlock + t + T * m];
-        if (NMAX > kJbBlock)  // the window's old and new places overlap
-            __syncthreads();
     }
     if (BITS == 32) {
         gu32 *o = reinterpret_cast<gu32 *>(G.out + (uint64_t)I.b * G.out_stride);
