@@ -397,7 +397,7 @@ def run_configs(M):
              substream_setup_first_ms=round(first_ms, 3),
              workload="4096 substreams i*3^162 of MTGP32-11213 set 0 (seed 777), 2^20 uint32 each, end to end: "
                       "substream start states made on the device as one matrix-core group (the 4095 states "
-                      "J^(i 3^162) w0 as fp4 products of the coefficient rows with the base window's bit planes; "
+                      "J^(i 3^162) w0 as fp4 products of coefficient blocks with the base window's bit planes, and their folds; "
                       "host time included, wall clock, median of 3 calls after the first, which also builds the "
                       "coefficient rows: substream_setup_first_ms) + generation")
     d["ms"] = round(setup_ms + jump_ms + gen_ms, 4)
@@ -463,8 +463,8 @@ def jump_latency(M, reps=20):
             r.fill(0, 1 << 20)
         out["reference_cpu_genrand_2^20_ms"] = round((time.perf_counter() - t) * 1e3 / 5, 4)
     out["what"] = ("one jump by 3^162 steps of MTGP32-11213 set 0 (2803-character string): fast_jump = the "
-                   "drop-in on a host mtgp32_fast_t (window up, the jump split over 11 waves by chunk range and "
-                   "their partial windows XORed by a second launch, window back, synchronous); "
+                   "drop-in on a host mtgp32_fast_t (window up, the products of its coefficient blocks on the "
+                   "matrix cores and their fold, window back, synchronous); "
                    "jump_poly = x^(3^162) mod P on the host; reference = the reference library on one core; "
                    "fill_ms = one mtgp32_fill of 2^k uint32 into a host array or a device buffer (window up, "
                    "launches of the plan built by the first call of that shape, window back, synchronous); "

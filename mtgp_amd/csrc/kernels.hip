@@ -1492,6 +1492,10 @@ __device__ __forceinline__ uint32_t transpose32(uint32_t v) {
     return v;
 }
 
+// These two kernels (bit planes of a whole sequence, then the products of all
+// its coefficients at once) were the matrix-core jumps before the blocked
+// ones of jump_blocks.hip, which run every jump now; only the emulated
+// kernel tests still call them.
 // One workgroup of kPlaneWaves waves per MJumpGroup: the base window (n
 // words), then the recursion 256 words at a time (one word per thread) in a
 // linear LDS buffer, relocated as in the generation kernels; every complete

@@ -1875,10 +1875,10 @@ void Plan::run_launches(int part, int phase, hipStream_t s) {
 // spread unevenly over the SIMDs: of 12 or 16 workgroups per CU, a fifth of the
 // CUs get one SIMD with one wave too many, which a long launch waits for.
 // After even a short launch of one-wave workgroups the next is spread evenly.
-// Measured: the batched MTGP32-11213 generation launch 3.64 -> 3.55 ms, 4096
-// cells of 2^20 numbers 3.96 -> 3.57 ms, for 2 to 3 us, which launches of
-// kSettleNumbers gain back.  (Two-wave cells gain nothing: 3.31 ms either way
-// for the MTGP64-23209 batch.)
+// Measured in layout 1: the batched MTGP32-11213 generation launch 3.64 ->
+// 3.55 ms, 4096 cells of 2^20 numbers 3.96 -> 3.57 ms, for 2 to 3 us, which
+// launches of kSettleNumbers gain back.  (Two-wave cells gain nothing: 3.31 ms
+// either way for the MTGP64-23209 batch.)
 constexpr uint64_t kSettleNumbers = (uint64_t)1 << 24;
 bool Plan::settles(const Launch &L) const {
     return layout_waves(L.layout) == 1 && L.numbers >= kSettleNumbers && L.grid >= 4 * ctx->cus;

@@ -162,7 +162,7 @@ struct Context {
     size_t fill_hcap = 0;
     // The shape fill_plan was built for.  A call of the same shape launches
     // it again without planning: its cells, jumps and output addresses do
-    // not depend on the start window, which the planes and jump kernels
+    // not depend on the start window, which the jump kernels
     // read when they run.
     struct FillShape {
         int slot = -1, bits = 0, kind = -1;
