@@ -270,19 +270,20 @@ int Context::per_cu(int bits, int cls, int layout, int cells, int knob) const {
     return b;
 }
 
-int Context::layout_one_round_for(int bits, int cls, int mask, int cells, uint64_t cell, uint64_t numbers) const {
+int Context::layout_one_round_for(int bits, int cls, int mask, int cells, uint64_t cell, uint64_t numbers,
+                                  double *ns) const {
     const int fixed = layout_one_round[bits == 64][cls];
-    if (fixed >= 0)
-        return layout_within(fixed, mask);
-    int best = 1;
-    double t = gen_ns(*this, bits, cls, 1, cells, cell, numbers);
-    for (int lay = 2; lay < kLayouts; lay++) {
+    int best = fixed >= 0 ? layout_within(fixed, mask) : 1;
+    double t = gen_ns(*this, bits, cls, best, cells, cell, numbers);
+    for (int lay = 2; fixed < 0 && lay < kLayouts; lay++) {
         if (!(mask >> lay & 1))
             continue;
         const double tl = gen_ns(*this, bits, cls, lay, cells, cell, numbers);
         if (tl < t)
             best = lay, t = tl;
     }
+    if (ns)
+        *ns = t;
     return best;
 }
 
@@ -954,65 +955,85 @@ double gen_ns(const Context &c, int bits, int cls, int layout, int cells, uint64
     if (rounds > 1)
         rate = lay == 1 ? 4700 : lay == 2 ? 4950 : 5100;
     const double t_store = (double)numbers * (bits / 8) / rate;
-    const double t = std::pow(std::pow(t_chain, 6) + std::pow(t_store, 6), 1.0 / 6);
+    auto cube = [](double v) { return v * v * v; };
+    const double t = std::cbrt(std::hypot(cube(t_chain), cube(t_store)));  // the 6-norm
     return rounds > 1 ? std::hypot(t, 10.0 * cells) : t;
+}
+
+// Cells of at least 4096 numbers, in whole wave steps.
+static uint64_t cell_size(double v) { return std::max<uint64_t>(((uint64_t)std::ceil(v) + 255) & ~255ull, 4096); }
+
+std::vector<uint64_t> one_round_sizes(const Context &c, uint64_t total_numbers, const std::vector<GridGroup> &groups,
+                                      int slots) {
+    uint64_t longest = 0;
+    int gens = 0;
+    for (const GridGroup &g : groups) {
+        gens += (int)g.numbers.size();
+        for (uint64_t v : g.numbers)
+            longest = std::max(longest, v);
+    }
+    std::vector<uint64_t> sizes;
+    auto add = [&](double v) {
+        sizes.push_back(cell_size(v));
+    };
+    for (double m = 1; m <= (double)slots && (double)longest / m > 4096 / 1.2; m = std::max(m + 1, std::floor(m * 1.15)))
+        add((double)longest / m);
+    for (int w = 1; w <= std::max(1, slots / std::max(1, c.cus)); w++)
+        add((double)total_numbers / std::max(1.0, (double)w * c.cus - 0.5 * (double)gens));
+    std::sort(sizes.begin(), sizes.end(), std::greater<uint64_t>());
+    sizes.erase(std::unique(sizes.begin(), sizes.end()), sizes.end());
+    // (beyond the longest stream every size is one cell per generator)
+    const auto first = std::partition_point(sizes.begin(), sizes.end(), [&](uint64_t S) { return S >= longest; });
+    if (first != sizes.begin())
+        sizes.erase(sizes.begin(), first - 1);
+    return sizes;
+}
+
+double one_round_ns(const Context &c, const std::vector<GridGroup> &groups, uint64_t S, int64_t &cells) {
+    double t = 0, floor_ns = 0;
+    cells = 0;
+    for (const GridGroup &g : groups) {
+        uint64_t count = 0, numbers = 0, top = 0;
+        // Jumps as the products see them: a generator's columns
+        // (one per jump and 1024 coefficients) in tiles of 32.
+        // (1000 MTGP64 dynamic-creator generators of one jump each:
+        // 190 ns a jump, 64 of 65 jumps 57 ns.)
+        const uint64_t ch = ((uint64_t)g.mexp + 1023) / 1024;
+        double jumps = 0;
+        for (uint64_t v : g.numbers) {
+            const uint64_t parts = (v + S - 1) / S;
+            jumps += (double)(((parts - 1) * ch + 31) / 32 * 32) / (double)ch;
+            count += parts;
+            numbers += v;
+            top = std::max(top, v);
+        }
+        const int n = (int)std::min<uint64_t>(count, INT32_MAX);
+        if (jumps > 0) {
+            t += jumps * (3.1e-7 * (double)g.mexp + 6e-4) * (double)g.mexp;
+            floor_ns = std::max(floor_ns, 0.75 * (double)g.mexp);
+        }
+        const uint64_t cell = std::min(S, top);
+        double gen = 0;
+        c.layout_one_round_for(g.bits, g.cls, g.layouts, n, cell, numbers, &gen);
+        t += gen;
+        cells += n;
+    }
+    return floor_ns > 0 ? t + floor_ns + c.jump_floor_ms * 1e6 : t;
 }
 
 bool auto_grid(const Context &c, uint64_t total_numbers, int n_requests, const std::vector<GridGroup> &groups, int slots,
                double jump_cost, double cell_waves, uint64_t &S1, uint64_t &S2, double &frac) {
     const double usable = std::max(1.0, (double)slots - (double)n_requests);
-    auto round256 = [](double v) { return std::max<uint64_t>(((uint64_t)v + 255) & ~255ull, 4096); };
     const double rho = jump_cost / std::max(1.0, (double)total_numbers / usable);
     if (rho > c.two_size_rho) {
         // One round of equal cells of the size with the least modelled step
-        // time.  Candidates: the longest stream in 1, 2, 3, ... parts (one
-        // part = no jumps at all), and 1 to 12 cells per CU over all of them
-        // (each generator's last cell is on average half full).
-        uint64_t longest = 0;
-        int gens = 0;
-        for (const GridGroup &g : groups) {
-            gens += (int)g.numbers.size();
-            for (uint64_t v : g.numbers)
-                longest = std::max(longest, v);
-        }
-        std::vector<uint64_t> sizes;
-        for (double m = 1; m <= (double)slots && (double)longest / m > 4096 / 1.2; m = std::max(m + 1, std::floor(m * 1.15)))
-            sizes.push_back(round256(std::ceil((double)longest / m)));
-        for (int w = 1; w <= std::max(1, slots / std::max(1, c.cus)); w++)
-            sizes.push_back(
-                round256(std::ceil((double)total_numbers / std::max(1.0, (double)w * c.cus - 0.5 * (double)gens))));
+        // time.
+        const std::vector<uint64_t> sizes = one_round_sizes(c, total_numbers, groups, slots);
         double best = -1;
         for (uint64_t S : sizes) {
-            double t = 0, floor_ns = 0;
-            int all = 0;
-            for (const GridGroup &g : groups) {
-                uint64_t cells = 0, numbers = 0, top = 0;
-                // Jumps as the products see them: a generator's columns
-                // (one per jump and 1024 coefficients) in tiles of 32.
-                // (1000 MTGP64 dynamic-creator generators of one jump each:
-                // 190 ns a jump, 64 of 65 jumps 57 ns.)
-                const uint64_t ch = ((uint64_t)g.mexp + 1023) / 1024;
-                double jumps = 0;
-                for (uint64_t v : g.numbers) {
-                    const uint64_t parts = (v + S - 1) / S;
-                    jumps += (double)(((parts - 1) * ch + 31) / 32 * 32) / (double)ch;
-                    cells += parts;
-                    numbers += v;
-                    top = std::max(top, v);
-                }
-                const int n = (int)std::min<uint64_t>(cells, INT32_MAX);
-                if (jumps > 0) {
-                    t += jumps * (3.1e-7 * (double)g.mexp + 6e-4) * (double)g.mexp;
-                    floor_ns = std::max(floor_ns, 0.75 * (double)g.mexp);
-                }
-                const uint64_t cell = std::min(S, top);
-                t += gen_ns(c, g.bits, g.cls, c.layout_one_round_for(g.bits, g.cls, g.layouts, n, cell, numbers), n, cell,
-                            numbers);
-                all += n;
-            }
-            if (floor_ns > 0)
-                t += floor_ns + c.jump_floor_ms * 1e6;
-            if (all > slots && S < longest)
+            int64_t cells;
+            const double t = one_round_ns(c, groups, S, cells);
+            if (cells > slots && S != sizes.front())
                 continue;
             if (best < 0 || t < best) {
                 best = t;
@@ -1033,8 +1054,8 @@ bool auto_grid(const Context &c, uint64_t total_numbers, int n_requests, const s
         S1 = S2 = auto_segment(c, total_numbers, n_requests, wslots);
         return false;
     }
-    S1 = round256(std::ceil(frac * (double)total_numbers / wusable));
-    S2 = round256(std::ceil((1 - frac) * (double)total_numbers / (wusable * c.small_rounds)));
+    S1 = cell_size(frac * (double)total_numbers / wusable);
+    S2 = cell_size((1 - frac) * (double)total_numbers / (wusable * c.small_rounds));
     return false;
 }
 

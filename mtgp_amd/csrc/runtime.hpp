@@ -207,7 +207,9 @@ struct Context {
     // are up to half a round more and the occupancy limit allows them.
     int per_cu(int bits, int cls, int layout, int cells, int knob) const;
     // The layout of a one-round launch (layout_one_round).
-    int layout_one_round_for(int bits, int cls, int mask, int cells, uint64_t cell, uint64_t numbers) const;
+    // Its modelled time (gen_ns) to *ns.
+    int layout_one_round_for(int bits, int cls, int mask, int cells, uint64_t cell, uint64_t numbers,
+                             double *ns = nullptr) const;
     void sha1_of(int slot, unsigned char out[20]) const;
 };
 
@@ -258,6 +260,14 @@ struct GridGroup {
 // times of 64 to 3072 cells in every class).  Beyond one round every cell is
 // claimed, 10 ns each on one counter.
 double gen_ns(const Context &c, int bits, int cls, int layout, int cells, uint64_t cell, uint64_t numbers);
+// The cell sizes that a one-round grid is chosen from, each once, largest
+// first: the longest stream in 1, 2, 3, ... parts (one part = no jumps at
+// all; the largest size is that one), and 1 to 12 cells per CU over all of them
+// (each generator's last cell is on average half full).
+std::vector<uint64_t> one_round_sizes(const Context &c, uint64_t total_numbers, const std::vector<GridGroup> &groups,
+                                      int slots);
+// The modelled time of a one-round grid of cells of S numbers, and its cells.
+double one_round_ns(const Context &c, const std::vector<GridGroup> &groups, uint64_t S, int64_t &cells);
 // Cell sizes for automatic segmentation: S1 for the first `frac` of each
 // generator's positions, S2 after (frac = 0: one size).  `jump_cost` is the
 // numbers-weighted mean jump_cost_numbers of the plan's generators: when a
