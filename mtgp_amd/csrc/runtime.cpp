@@ -636,7 +636,9 @@ JumpCache::JumpCache(Context &c, const std::vector<int> &slots, uint64_t cell, i
         list.push_back(&entries_[s]);
     // One task per (slot, block of table entries): the table is a chain of
     // products, so each block starts from its own x^(k0 cell).
-    constexpr uint64_t kBlock = 64;
+    // (a block's start costs about 6 products; shorter blocks where there are
+    // few, so that they still spread over the pool)
+    const uint64_t kBlock = list.size() * (B_ / 64) >= 16 ? 64 : 16;
     const uint64_t nblocks = (B_ + kBlock - 1) / kBlock;
     parallel_for((int)list.size(), [&](int i) {
         Entry &e = *list[(size_t)i];
@@ -683,6 +685,11 @@ std::shared_ptr<JumpCache> JumpCache::shared(Context &c, const std::vector<int> 
     auto it = g_caches.find(key);
     if (it != g_caches.end())
         return it->second;
+    if (!far)  // a longer table serves as well
+        for (const auto &e : g_caches)
+            if (std::get<0>(e.first) == c.device && std::get<1>(e.first) == cell && std::get<2>(e.first) < -kmax &&
+                std::get<3>(e.first) == keys)
+                return e.second;
     // at most kMaxCaches kept: drop the ones nobody else holds
     constexpr size_t kMaxCaches = 32;
     if (g_caches.size() >= kMaxCaches)
@@ -770,9 +777,9 @@ size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 double jump_cost_numbers(int mexp, int n) { return 0.026 * (double)mexp * (double)n; }
 
-// Plans on a uniform grid with a generator of at least kAutoCacheCells
-// cells take their jump polynomials from a process-wide JumpCache of
-// kAutoCacheCells * 2^i entries, up to kAutoCacheMaxK.
+// Plans on a uniform grid take the jump polynomials of generators of at least
+// kAutoCacheCells cells (2 on a table_cell grid) from a process-wide JumpCache,
+// up to kAutoCacheMaxK cells.
 constexpr int kAutoCacheCells = 64;
 constexpr int kAutoCacheMaxK = 2048;
 // Cells per block of an incremental polynomial chain on the host pool.
@@ -963,6 +970,16 @@ double gen_ns(const Context &c, int bits, int cls, int layout, int cells, uint64
 // Cells of at least 4096 numbers, in whole wave steps.
 static uint64_t cell_size(double v) { return std::max<uint64_t>(((uint64_t)std::ceil(v) + 255) & ~255ull, 4096); }
 
+uint64_t table_cell(uint64_t longest, int gens, uint64_t S) {
+    auto worth = [&](uint64_t cell) {
+        return gens == 1 ? longest / cell >= 2 : longest / cell >= (gens <= 16 ? 4u : 16u) && cell <= (uint64_t)1 << 17;
+    };
+    if (!worth(S))
+        return 0;
+    const uint64_t T = octave_size(S, gens == 1 ? 4 : 8);
+    return worth(T) ? T : 0;
+}
+
 std::vector<uint64_t> one_round_sizes(const Context &c, uint64_t total_numbers, const std::vector<GridGroup> &groups,
                                       int slots) {
     uint64_t longest = 0;
@@ -974,7 +991,9 @@ std::vector<uint64_t> one_round_sizes(const Context &c, uint64_t total_numbers, 
     }
     std::vector<uint64_t> sizes;
     auto add = [&](double v) {
-        sizes.push_back(cell_size(v));
+        const uint64_t S = cell_size(v);
+        const uint64_t T = table_cell(longest, gens, S);
+        sizes.push_back(T ? T : S);
     };
     for (double m = 1; m <= (double)slots && (double)longest / m > 4096 / 1.2; m = std::max(m + 1, std::floor(m * 1.15)))
         add((double)longest / m);
@@ -1113,6 +1132,7 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
     int slots = 0;
     double jcost = 0, weight = 0;
     std::vector<GridGroup> groups_of(7);
+    int gens_named = 0;  // with numbers to generate
     double cell_waves = 0;
     for (int g : named) {
         const GenRef &gr = gens[(size_t)g];
@@ -1131,6 +1151,7 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
         gg.layouts = group_ok[3 * b + cls];
         gg.mexp = std::max(gg.mexp, gr.mexp);
         gg.numbers.push_back(per[(size_t)g]);
+        gens_named++;
     }
     groups_of.erase(std::remove_if(groups_of.begin(), groups_of.end(), [](const GridGroup &g) { return g.numbers.empty(); }),
                     groups_of.end());
@@ -1255,16 +1276,20 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
     // A uniform grid (one cell size, no caller cache) with a generator of
     // many cells -- one long stream, as mtgp32_fill and the torch Generator
     // make -- takes its polynomials x^(k S) from a process-wide cache: a
-    // repeated request of the same size then needs no polynomial product,
-    // and the first builds the table in blocks on the host pool.
+    // request whose grid has the same cell size then needs no polynomial
+    // product, and the first builds the table in blocks on the host pool.
     std::shared_ptr<JumpCache> auto_cache;
     const JumpCache *cache = opt.cache;
     if (!cache && frac == 0 && S > 0) {
-        uint64_t kmax = 0;
+        uint64_t kmax = 0, longest = 0;
+        for (int g : named)
+            longest = std::max(longest, per[(size_t)g]);
+        const size_t least =
+            one_round && table_cell(longest, gens_named, S) == S ? 2 : (size_t)kAutoCacheCells;
         std::vector<int> slots;
         for (int g = 0; g < G; g++) {
             const auto &cv = cells[(size_t)g];
-            if (cv.size() < (size_t)kAutoCacheCells)
+            if (cv.size() < least)
                 continue;
             slots.push_back(gens[(size_t)g].slot);
             for (const Cell &cl : cv)
@@ -1272,10 +1297,7 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
                     kmax = std::max<uint64_t>(kmax, cl.start / S);
         }
         if (!slots.empty() && kmax <= (uint64_t)kAutoCacheMaxK) {
-            int k = kAutoCacheCells;
-            while ((uint64_t)k < kmax)
-                k *= 2;
-            auto_cache = JumpCache::shared(c, slots, S, k, false);
+            auto_cache = JumpCache::shared(c, slots, S, (int)octave_size(kmax, 4), false);
             cache = auto_cache.get();
         }
     }

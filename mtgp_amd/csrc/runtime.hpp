@@ -260,6 +260,24 @@ struct GridGroup {
 // times of 64 to 3072 cells in every class).  Beyond one round every cell is
 // claimed, 10 ns each on one counter.
 double gen_ns(const Context &c, int bits, int cls, int layout, int cells, uint64_t cell, uint64_t numbers);
+// The least m 2^k >= v with steps <= m < 2 steps.
+inline uint64_t octave_size(uint64_t v, uint64_t steps) {
+    uint64_t unit = 1;
+    while (unit * 2 * steps <= v)
+        unit *= 2;
+    return std::max<uint64_t>((v + unit - 1) / unit, steps) * unit;
+}
+// The cell size that a one-round grid takes for cells of S numbers so that its
+// jump polynomials x^(k T) are those of other lengths' grids too, and are kept
+// (JumpCache::shared); 0 = none, the exact one is better.  With exact sizes a
+// call of another length found no table and made one on the host (calls 0 to
+// 2% shorter than n, exact sizes and these: one MTGP32-23209 stream of 10^6
+// numbers 3.04 and 0.10 ms a call, two of 5 * 10^5 2.4 and 0.10 ms; one
+// MTGP64-110503 stream of 2^24 38 and 0.47 ms).  4 sizes an octave cost one
+// stream 0.7% of its modelled step time at most, on average over a decade of
+// lengths, 8 cost a few streams 1.5%; more streams or longer cells, whose
+// repeated calls would lose up to 7%, keep the exact sizes.
+uint64_t table_cell(uint64_t longest, int gens, uint64_t S);
 // The cell sizes that a one-round grid is chosen from, each once, largest
 // first: the longest stream in 1, 2, 3, ... parts (one part = no jumps at
 // all; the largest size is that one), and 1 to 12 cells per CU over all of them
@@ -290,7 +308,8 @@ class JumpCache {
     // far = false leaves out the tables for positions beyond kmax cells
     // (lookups there then fail and the planner computes those cells).
     JumpCache(Context &c, const std::vector<int> &slots, uint64_t cell, int kmax, bool far = true);
-    // One cache per (device, cell, kmax, slots) for the whole process.
+    // One cache per (device, cell, kmax, slots) for the whole process, or
+    // (far = false) one of a larger kmax.
     static std::shared_ptr<JumpCache> shared(Context &c, const std::vector<int> &slots, uint64_t cell, int kmax,
                                              bool far = true);
     uint64_t cell() const { return cell_; }

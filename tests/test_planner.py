@@ -1,7 +1,11 @@
 """The planner's choices on the CPU, against an MI355X's occupancy limits
-(tests/planner): which cell sizes a one-round grid is chosen from."""
+(tests/planner): which cell sizes a one-round grid is chosen from, and that
+streams of nearby lengths are cut alike, so that their jump polynomials are in
+the tables that an earlier call left.  Whole numbers throughout."""
 import ctypes as C
+import math
 import os
+import random
 import subprocess
 
 import pytest
@@ -34,6 +38,14 @@ def _sizes(lib, key, numbers):
     return list(out[:n])
 
 
+def _is_table_size(v, steps=4):
+    while v >= 2 * steps:
+        if v % 2:
+            return False
+        v //= 2
+    return v >= steps
+
+
 def _cell(lib, key, numbers):
     return lib.planner_cell(*_args(key, numbers))
 
@@ -49,3 +61,47 @@ def test_each_size_is_priced_once(lib, key):
         best = min(lib.planner_ns(*_args(key, numbers), s) for s in sizes
                    if s == sizes[0] or sum(-(-n // s) for n in numbers) <= 12 * 256)
         assert lib.planner_ns(*_args(key, numbers), _cell(lib, key, numbers)) == best
+
+
+@pytest.mark.parametrize("key", CLASSES)
+@pytest.mark.parametrize("n", [10**6, 1 << 24])
+def test_nearby_lengths_share_a_grid(lib, key, n):
+    """40 lengths of one stream within 2%: two cell sizes at most."""
+    rng = random.Random(n)
+    cells = {_cell(lib, key, [n - rng.randrange(n // 50)]) for _ in range(40)}
+    assert len(cells) <= 2, cells
+
+
+@pytest.mark.parametrize("key", CLASSES)
+def test_streams_of_many_cells_take_table_sizes(lib, key):
+    rng = random.Random(3)
+    for lo, hi in ((10**5, 10**6), (10**6, 10**7), (10**7, 10**8)):
+        cells = set()
+        for _ in range(60):
+            n = int(math.exp(rng.uniform(math.log(lo), math.log(hi))))
+            S = _cell(lib, key, [n])
+            assert n // S < 3 or _is_table_size(S), (n, S)  # (2 cells stay 2 or more)
+            if n // S >= 3:
+                cells.add(S)
+        assert len(cells) <= 14, cells  # 4 an octave over a decade
+
+
+@pytest.mark.parametrize("gens,parts", [(2, 4), (16, 4), (17, 16), (64, 16)])
+def test_sets_take_table_sizes_for_many_short_cells(lib, gens, parts):
+    """From `parts` cells each on, of 2^17 numbers at most; the rounding may
+    cost one cell in 9."""
+    n = 1 << 22 if gens < 17 else 1 << 20
+    sizes = _sizes(lib, (64, 0), [n + 1] * gens)
+    assert all(_is_table_size(s, 8) for s in sizes if n // s >= parts + parts // 4 and s <= 7 << 14)
+    assert any(not _is_table_size(s, 8) for s in sizes if 1 < n // s < parts), sizes
+    sizes = _sizes(lib, (64, 0), [1 << 25] * 64)
+    assert any(s > 1 << 17 and not _is_table_size(s, 8) for s in sizes)
+
+
+@pytest.mark.parametrize("key", CLASSES)
+@pytest.mark.parametrize("gens,n", [(2, 500000), (3, 2 * 10**6), (8, 400000)])
+def test_nearby_lengths_of_few_streams_share_a_grid(lib, key, gens, n):
+    rng = random.Random(n)
+    cells = {_cell(lib, key, [n - rng.randrange(n // 50)] * gens) for _ in range(40)}
+    cells = {S for S in cells if n // S >= 5 and S <= 7 << 14}
+    assert len(cells) <= 3, cells
