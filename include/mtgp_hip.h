@@ -233,10 +233,11 @@ void mtgp_plan_destroy(mtgp_plan_t *plan);
  * unchanged. */
 int mtgp_plan_configure(mtgp_plan_t *plan, int layout, int blocks_per_cu);
 /* Two-phase launch order (off by default; MTGP_OVERLAP=1 changes the
- * default): on the automatic two-size grid, mtgp_plan_launch runs the large
- * cells' jumps, then their generation on `stream` while the small cells'
- * jumps and generation run on a side stream of the plan, which `stream`
- * waits for at the end.  Returns 1 if the plan now launches in two phases,
+ * default): on the automatic two-size grid, mtgp_plan_launch runs the jumps
+ * of all cells, then the large cells' generation on `stream` beside the small
+ * cells' on a side stream of the plan, which `stream` waits for at the end.
+ * Jumps of the word-XOR kernel (jump_mfma_min = 0) are split: the large cells'
+ * first, the small cells' on the side stream.  Returns 1 if the plan now launches in two phases,
  * 0 if it launches serially (no small cells, or off), -1 on error. */
 int mtgp_plan_set_overlap(mtgp_plan_t *plan, int on);
 /* Enqueues one part of a plan, in serial order on `stream`: 0 = the

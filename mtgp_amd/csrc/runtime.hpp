@@ -112,9 +112,8 @@ struct Context {
     double two_size_rho = 0.15;
     double jump_floor_ms = 0.008;
     // Two-phase launches of two-size grids (MTGP_OVERLAP=1).  Off by
-    // default: on the batched MTGP32-11213 workload the side stream's jumps
-    // share the generation kernel's power budget rather than hide behind its
-    // stores (4.8 ms per step against 4.6 ms serial).
+    // default: even with the serial order (128 MTGP32-11213 streams of 2^22
+    // words 717 us against 734, 16 of 2^25 713 against 705).
     bool overlap = false;
     // Batched jumps are split into partial jumps (chunk ranges, XORed when
     // the generation kernel loads the start window) until a jump launch has
@@ -406,13 +405,15 @@ class JumpBlockList {
 //
 // Two-phase launch (overlap): with the two-size grid, the large cells (one
 // per resident workgroup, the first round) form phase 0 and the small cells
-// phase 1.  launch() runs phase 0's jumps, then phase 0's generation on the
-// caller's stream while phase 1's jumps, then phase 1's generation, run on
-// a side stream; the caller's stream waits for the side stream at the end.
-// Phase 1's jumps then run beside generation and phase 1's generation fills
-// phase 0's tail; measured on MI355X the jumps share the generation
-// kernel's power budget instead of hiding behind it, so the order is off by
-// default (set_overlap).  launch_part runs the merged launches (one jump
+// phase 1.  launch() runs the blocked jumps of both (and phase 0's word-XOR
+// ones), then phase 0's generation on the caller's stream beside phase 1's
+// (after its word-XOR jumps) on a side stream; the caller's stream waits for
+// the side stream at the end.  Even with the serial order, so off by default
+// (set_overlap); phase 1's blocked jumps beside generation were slower (128
+// MTGP32-11213 streams of 2^22 words 771 us against 717, 64 MTGP32-23209
+// ones 848 against 817; MTGP64 dynamic-creator sets alone gained, 1012
+// against 1060): they take the LDS and the power that generation runs on.
+// launch_part runs the merged launches (one jump
 // and one generation launch per class over both phases: the serial order).
 struct Plan {
     struct Launch {
