@@ -270,6 +270,24 @@ int Context::per_cu(int bits, int cls, int layout, int cells, int knob) const {
     return b;
 }
 
+int Context::launch_per_cu(int bits, int cls, int layout, int cells, bool one_round) const {
+    if (one_round)
+        return per_cu(bits, cls, layout, cells, bpc[bits == 64][cls]);
+    const int knob = rounds_knob(bits, cls, layout, cells);
+    if (rounds_tuned[bits == 64][cls][layout] > 0)
+        return std::min(knob, blocks_per_cu[bits == 64][cls][layout]);
+    return per_cu(bits, cls, layout, cells, knob);
+}
+
+void Context::keep_tuned(int bits, int cls, int layout, int per_cu, bool one_round, bool whole) {
+    if (one_round)
+        bpc[bits == 64][cls] = per_cu;
+    else
+        rounds_tuned[bits == 64][cls][layout] = per_cu;
+    if (whole)
+        (one_round ? layout_one_round : this->layout)[bits == 64][cls] = layout;
+}
+
 int Context::layout_one_round_for(int bits, int cls, int mask, int cells, uint64_t cell, uint64_t numbers,
                                   double *ns) const {
     const int fixed = layout_one_round[bits == 64][cls];
@@ -1758,9 +1776,7 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
                     gen_ns(c, L.bits, L.cls, 1, L.count, longest, L.numbers) <
                         gen_ns(c, L.bits, L.cls, L.layout, L.count, longest, L.numbers))
                     L.layout = 1;
-                const int bpc = c.per_cu(
-                    L.bits, L.cls, L.layout, L.count,
-                    fits ? knob : c.rounds_knob(L.bits, L.cls, L.layout, L.count));
+                const int bpc = c.launch_per_cu(L.bits, L.cls, L.layout, L.count, fits);
                 L.grid = std::min(L.count, c.cus * bpc);
                 L.dyn_lds = c.lds_reserve(kernel_fn(L.bits, L.cls, L.layout), kernel_threads(L.bits, L.cls, L.layout), bpc);
             }
@@ -2041,11 +2057,8 @@ float Plan::autotune(hipStream_t s, int reps, int *best_layout, int *best_bpc) {
     configure(bl, bb);
     std::unique_lock<std::shared_mutex> tune_lock(ctx->tune_mu);
     ctx->tune_epoch++;
-    for (const auto &L : launches) {
-        if (L.layout == bl)
-            (one_round_grid ? ctx->layout_one_round : ctx->layout)[L.bits == 64][L.cls] = bl;
-        ctx->bpc[L.bits == 64][L.cls] = bb;
-    }
+    for (const auto &L : launches)
+        ctx->keep_tuned(L.bits, L.cls, L.layout, bb, one_round_grid, L.layout == bl);
     if (best_layout)
         *best_layout = bl;
     if (best_bpc)

@@ -52,10 +52,22 @@ struct Context {
     // MTGP32-11213 cells of 17 GB 3576, 3384 and 3352, 3314 us; 6000, 8192
     // 3155, 3126 and 3246, 3158; 4096 of MTGP32-23209 3226 and 3139).
     int rounds_knob(int bits, int cls, int layout, int cells) const {
+        if (rounds_tuned[bits == 64][cls][layout] > 0)
+            return rounds_tuned[bits == 64][cls][layout];
         const int knob = bpc[bits == 64][cls], share = layout == 3 ? (bits == 64 && cls == 1 ? 4 : 2) : layout == 2 ? 2 : 1;
         const int cap = std::min(knob, blocks_per_cu[bits == 64][cls][layout]);
         return layout == 3 && share == 2 && cells <= 2 * cus * cap ? cap : std::max(1, knob / share);
     }
+    // The autotuner's for each layout, as it measured them; 0 = not tuned.
+    int rounds_tuned[2][4][4] = {};
+    // Workgroups per CU of a generation launch, on a one-round grid or any
+    // other.
+    int launch_per_cu(int bits, int cls, int layout, int cells, bool one_round) const;
+    // Makes per_cu (and the layout, if `whole`) the default of later launches
+    // of the class: a grid of several rounds is sized by bpc and run by
+    // rounds_tuned, so that a later plan of the same requests is the one that
+    // was measured.
+    void keep_tuned(int bits, int cls, int layout, int per_cu, bool one_round, bool whole);
     // The layout whose occupancy and waves size the cells of such grids: more
     // cells would cost more jumps than the even finish gains (the two-size
     // grid of the batched MTGP32-11213 workload for 6, 8 and 12 cells per CU
@@ -77,8 +89,8 @@ struct Context {
     // against 4.60-4.63 ms at 16 and 4.71 ms at 8.
     int default_bpc = 12;
     // Resident workgroups per CU for generation launches per [bits==64][class]
-    // (until the autotuner measures better; MTGP_BLOCKS_PER_CU sets them
-    // all).  default_bpc everywhere but the MTGP64 128-word-step class
+    // (until the autotuner measures better on a one-round grid;
+    // MTGP_BLOCKS_PER_CU sets them all).  default_bpc everywhere but the MTGP64 128-word-step class
     // (dynamic-creator sets, N = 176): 8, which halves the cells' jumps
     // there; its 64-set batch measured 4207-4212 GB/s per step at 8
     // against 4032-4041 at 12 and 3557-3574 at 16, while the other classes

@@ -52,6 +52,17 @@ double planner_ns(int bits, int cls, int mexp, int n, const uint64_t *numbers, u
     return one_round_ns(*c, group(bits, cls, mexp, n, numbers), cell, cells);
 }
 
+// Workgroups per CU of a later launch of `cells` cells in the class's default
+// layout (to *layout), after the autotuner chose (tuned_layout, tuned).
+int planner_tuned(int bits, int cls, int tuned_layout, int tuned, int one_round, int cells, int *layout) {
+    std::unique_ptr<Context> c(make());
+    c->keep_tuned(bits, cls, tuned_layout, tuned, one_round != 0, true);
+    const int mask = bits == 64 && cls == 3 ? 3 : 15;
+    *layout = one_round ? c->layout_one_round_for(bits, cls, mask, cells, 1 << 16, (uint64_t)cells << 16)
+                        : c->layout_for(bits, cls, mask);
+    return c->launch_per_cu(bits, cls, *layout, cells, one_round != 0);
+}
+
 // The one-round grid's cell size.
 uint64_t planner_cell(int bits, int cls, int mexp, int n, const uint64_t *numbers) {
     std::unique_ptr<Context> c(make());

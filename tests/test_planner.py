@@ -1,7 +1,8 @@
 """The planner's choices on the CPU, against an MI355X's occupancy limits
-(tests/planner): which cell sizes a one-round grid is chosen from, and that
+(tests/planner): which cell sizes a one-round grid is chosen from, that
 streams of nearby lengths are cut alike, so that their jump polynomials are in
-the tables that an earlier call left.  Whole numbers throughout."""
+the tables that an earlier call left, and that an autotuned launch shape is
+the one that later plans run.  Whole numbers throughout."""
 import ctypes as C
 import math
 import os
@@ -12,6 +13,9 @@ import pytest
 
 HERE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "planner")
 U64 = C.c_uint64
+# Workgroups per CU that fit, by layout (as tests/planner/driver.cpp has them)
+LIMITS = {(32, 0): (32, 32, 16, 8), (32, 1): (24, 24, 16, 8), (32, 2): (16, 16, 13, 4), (64, 0): (16, 16, 15, 7),
+          (64, 1): (13, 13, 8, 7), (64, 2): (7, 7, 5, 3), (64, 3): (30, 30, 30, 30)}
 # (word size, state class): MEXP
 CLASSES = {(32, 0): 11213, (32, 1): 23209, (32, 2): 44497, (64, 0): 23209, (64, 1): 44497, (64, 2): 110503, (64, 3): 3217}
 
@@ -105,3 +109,16 @@ def test_nearby_lengths_of_few_streams_share_a_grid(lib, key, gens, n):
     cells = {_cell(lib, key, [n - rng.randrange(n // 50)] * gens) for _ in range(40)}
     cells = {S for S in cells if n // S >= 5 and S <= 7 << 14}
     assert len(cells) <= 3, cells
+
+
+@pytest.mark.parametrize("key", CLASSES)
+def test_later_launches_run_what_the_autotuner_measured(lib, key):
+    """Every (layout, workgroups per CU) that the tuner tries, over launches of
+    several rounds: at, below and beyond two rounds of it."""
+    for layout in (1,) if key == (64, 3) else (0, 1, 2, 3):
+        for per_cu in (2, 4, 6, 8, 12, 16):
+            got = C.c_int()
+            for cells in (256 * per_cu + 1, 300 * per_cu, 512 * per_cu, 512 * per_cu + 1, 5000 * per_cu):
+                n = lib.planner_tuned(*key, layout, per_cu, 0, cells, C.byref(got))
+                assert got.value == layout
+                assert n == min(per_cu, LIMITS[key][layout]), (layout, per_cu, cells)
