@@ -945,6 +945,10 @@ void JumpBlockList::run(const Context &c, const char *d, const JumpBlocks *g, hi
     }
 }
 
+JumpSpace::JumpSpace(size_t list_bytes, size_t coef_bytes, size_t window_bytes, size_t part_bytes)
+    : o_coef(align256(list_bytes)), o_in(o_coef + align256(coef_bytes)), o_out(o_in + align256(window_bytes)),
+      o_parts(o_out + align256(window_bytes)), device_bytes(o_parts + part_bytes), host_bytes(o_parts) {}
+
 double gen_ns(const Context &c, int bits, int cls, int layout, int cells, uint64_t cell, uint64_t numbers) {
     // ns per number of a cell alone on its CU, layouts 1 to 3 (64 cells of
     // 64 generators; the longest state a class has in the tables).
@@ -2132,9 +2136,8 @@ struct mtgp_plan {
 };
 
 // One jump in coefficient blocks: the block lists, coefficients and (host_io)
-// the window go up in one copy to the context's workspace [lists |
-// coefficients | window in | partial windows | window out], two launches, the
-// window back.  False (nothing done) when the partial windows of a very long
+// the window go up in one copy to the context's workspace (JumpSpace), two
+// launches, the window back.  False (nothing done) when the partial windows of a very long
 // polynomial would outgrow a round's memory.
 static bool device_jump_blocks(Context &c, int slot, int bits, int mexp, const void *in, void *out,
                                const std::vector<uint32_t> &words, bool host_io) {
@@ -2150,14 +2153,11 @@ static bool device_jump_blocks(Context &c, int slot, int bits, int mexp, const v
     L.add(c, slot, host_io ? 0 : (uint64_t)(uintptr_t)in, 0, (int)blocks, 1, host_io ? 0 : (uint64_t)(uintptr_t)out,
           wbytes);
     L.finish(c.cus);
-    const size_t o_coef = L.list_bytes();
-    const size_t o_in = o_coef + align256(blocks * kJbWords * 4);
-    const size_t o_parts = o_in + align256(wbytes);
-    const size_t o_out = o_parts + L.part_bytes();
-    const size_t need = o_out + align256(wbytes);
+    const JumpSpace W(L.list_bytes(), blocks * kJbWords * 4, wbytes, L.part_bytes());
+    const size_t o_coef = W.o_coef, o_in = W.o_in, o_out = W.o_out, o_parts = W.o_parts;
     std::lock_guard<std::mutex> lk(c.jump_mu);
-    grow_device(c.jump_d, c.jump_dcap, need, "hipMalloc jump workspace");
-    grow_pinned(c.jump_h, c.jump_hcap, need);
+    grow_device(c.jump_d, c.jump_dcap, W.device_bytes, "hipMalloc jump workspace");
+    grow_pinned(c.jump_h, c.jump_hcap, W.host_bytes);
     char *d = c.jump_d, *h = c.jump_h;
     const uint64_t dw = (uint64_t)(uintptr_t)d;
     L.relocate(dw + o_coef, dw + o_parts, host_io ? dw + o_out : 0);

@@ -406,6 +406,14 @@ class JumpBlockList {
     bool fresh_ = true;
 };
 
+// The workspace of one jump in coefficient blocks: [lists | coefficients |
+// window in | window out | partial windows], of which the host stages all but
+// the partial windows (29 MB for 10^7 coefficients of an MTGP64-23209 jump).
+struct JumpSpace {
+    size_t o_coef, o_in, o_out, o_parts, device_bytes, host_bytes;
+    JumpSpace(size_t list_bytes, size_t coef_bytes, size_t window_bytes, size_t part_bytes);
+};
+
 // A list of device Items plus the launches that run them.
 //
 // Each generator's requests occupy consecutive positions of its stream

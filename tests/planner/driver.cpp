@@ -63,6 +63,14 @@ int planner_tuned(int bits, int cls, int tuned_layout, int tuned, int one_round,
     return c->launch_per_cu(bits, cls, *layout, cells, one_round != 0);
 }
 
+// Offsets and sizes of a jump's workspace.
+void planner_jump_space(const uint64_t *bytes, uint64_t *out) {
+    const JumpSpace W(bytes[0], bytes[1], bytes[2], bytes[3]);
+    const uint64_t v[] = {W.o_coef, W.o_in, W.o_out, W.o_parts, W.device_bytes, W.host_bytes};
+    for (int k = 0; k < 6; k++)
+        out[k] = v[k];
+}
+
 // The one-round grid's cell size.
 uint64_t planner_cell(int bits, int cls, int mexp, int n, const uint64_t *numbers) {
     std::unique_ptr<Context> c(make());

@@ -122,3 +122,14 @@ def test_later_launches_run_what_the_autotuner_measured(lib, key):
                 n = lib.planner_tuned(*key, layout, per_cu, 0, cells, C.byref(got))
                 assert got.value == layout
                 assert n == min(per_cu, LIMITS[key][layout]), (layout, per_cu, cells)
+
+
+@pytest.mark.parametrize("lists,coef,window,parts", [(256, 128, 1404, 1408), (256, 1408, 1404, 15488),
+                                                     (512, 4000 * 128, 13816, 4000 * 13824), (256, 1, 1, 128 << 20)])
+def test_the_host_stages_no_partial_windows(lib, lists, coef, window, parts):
+    out = (U64 * 6)()
+    lib.planner_jump_space((U64 * 4)(lists, coef, window, parts), out)
+    o_coef, o_in, o_out, o_parts, device, host = out
+    assert all(o % 256 == 0 for o in (o_coef, o_in, o_out, o_parts))
+    assert lists <= o_coef and o_coef + coef <= o_in and o_in + window <= o_out and o_out + window <= o_parts
+    assert device == o_parts + parts and host <= lists + coef + 2 * window + 4 * 256
