@@ -17,6 +17,7 @@ so no other GPU framework needs to be loaded into the process.  If the
 library has not been built, importing this package raises ImportError.
 """
 import ctypes as C
+import functools
 import os
 import struct
 
@@ -524,6 +525,14 @@ class GenSet:
 
 
 _PACKED = "iiQQP"  # mtgp_request_t
+# Requests packed at once: each count below needs a compiled format of its own
+# (5 entries of 32 bytes per request), which are kept.
+_PACK_BLOCK = 128
+
+
+@functools.lru_cache(maxsize=_PACK_BLOCK)
+def _packer(n):
+    return struct.Struct(_PACKED * n)
 
 
 def _request_array(n, fields, plain=True):
@@ -532,7 +541,9 @@ def _request_array(n, fields, plain=True):
     try:
         if not plain:
             raise struct.error
-        struct.pack_into(_PACKED * n, arr, 0, *fields)
+        for k in range(0, n, _PACK_BLOCK):
+            m = min(_PACK_BLOCK, n - k)
+            _packer(m).pack_into(arr, C.sizeof(Request) * k, *fields[5 * k:5 * (k + m)])
     except struct.error:  # negative or wide numbers, None: as ctypes converts them
         for k in range(n):
             arr[k].gen, arr[k].kind, arr[k].count, arr[k].skip, arr[k].out = fields[5 * k:5 * k + 5]
