@@ -73,8 +73,9 @@ struct alignas(16) JumpItem {
 };
 static_assert(sizeof(JumpItem) == 64, "JumpItem layout");
 
-// Jumps on the matrix cores: nj jumps of one MTGP32 base window, as one
-// GF(2) product of their coefficient bits with the bit planes of the base's
+// Jumps on the matrix cores in one product (run by the kernel emulation only;
+// jump_blocks.hpp has those of the library): nj jumps of one MTGP32 base
+// window, as one GF(2) product of their coefficient bits with the bit planes of the base's
 // sequence (kernels.hip, mtgp32_jump_mfma_kernel).
 //  - planes : 32 * pw words the planes kernel fills (positions [0, 32 pw)).
 //  - coef   : coefficient words, coef[w * njp + b] = word w of jump b

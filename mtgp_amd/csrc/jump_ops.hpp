@@ -71,9 +71,11 @@ __device__ __forceinline__ void swap_halves(uint32_t &a, uint32_t &b) {
     b = r[1];
 }
 
-// acc + A B with A 32 x 64 and B 64 x 32 in fp4 (the operand and result
-// layout of mfma_fp4_32x32x64), in the form without block scales: an 8-byte
-// instruction with no scale registers.
+// acc + A B with A 32 x 64 and B 64 x 32 in fp4: lane L holds row L % 32 of A
+// and column L % 32 of B, both for the 32 values of K group L / 32 (the same
+// value index means the same k in both); acc[r] of lane L is row 8 (r / 4) +
+// 4 (L / 32) + r % 4, column L % 32.  In the form without block scales: an
+// 8-byte instruction with no scale registers.
 __device__ __forceinline__ mfma_v16f mfma_bits_32x32x64(mfma_v8i a, mfma_v8i b, mfma_v16f acc) {
     return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, acc, 4, 4, 0, 0, 0, 0);
 }

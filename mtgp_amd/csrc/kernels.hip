@@ -1435,7 +1435,12 @@ hipError_t launch_combine(const JumpItem *items, int n_items, hipStream_t s) {
     return hipGetLastError();
 }
 
-// ------------------------------------------------- jumps on the matrix cores
+// --------------------------------- jumps on the matrix cores, in one product
+// The matrix-core jumps before the blocked ones of jump_blocks.hip: bit planes
+// of a whole sequence, then the products of all its coefficients at once.  No
+// launch reaches them and the library does not hold them; the kernel
+// emulation, built as plain C++, still runs them against the oracle.
+#ifndef __HIP__
 // The nj jumps of one base window are one GF(2) product: bit p of jump b's
 // new word j is the parity of sum_k c_b[k] * bit_p(w[k + j]) over the
 // base's sequence w (the fold of mtgp32_jump_kernel, one bit at a time).
@@ -1492,10 +1497,6 @@ __device__ __forceinline__ uint32_t transpose32(uint32_t v) {
     return v;
 }
 
-// These two kernels (bit planes of a whole sequence, then the products of all
-// its coefficients at once) were the matrix-core jumps before the blocked
-// ones of jump_blocks.hip, which run every jump now; only the emulated
-// kernel tests still call them.
 // One workgroup of kPlaneWaves waves per MJumpGroup: the base window (n
 // words), then the recursion 256 words at a time (one word per thread) in a
 // linear LDS buffer, relocated as in the generation kernels; every complete
@@ -1684,5 +1685,6 @@ hipError_t launch_jump_mfma32(const MJumpGroup *groups, const MJumpItem *items, 
     hipLaunchKernelGGL(fn, dim3(n_items), dim3(kWave), 0, s, groups, items);
     return hipGetLastError();
 }
+#endif
 
 }  // namespace mtgp

@@ -48,7 +48,8 @@ const void *jump_kernel_fn(int bits, int cls);
 hipError_t launch_jumps(int bits, int cls, const JumpItem *items, int n_items, const DevParam *params,
                         uint32_t *queue, int grid, size_t dyn_lds, hipStream_t s);
 
-// Matrix-core jumps (MJumpGroup, common.hpp), MTGP32 sets with n <= 1391
+// Matrix-core jumps in one product (the kernel emulation only; MJumpGroup,
+// common.hpp), MTGP32 sets with n <= 1391
 // and n - pos >= 256: first the bit planes of every group (one workgroup per
 // group), then the products (one workgroup per MJumpItem; every item of a
 // launch has jumps in exactly row_tiles of its 32-jump row tiles, 1..2).
