@@ -649,17 +649,23 @@ def cpu_config_baselines(seconds=3.0):
     return out
 
 
-def measured_traffic(path=os.path.join(ROOT, "profiles", "mtgp32_items_batched11213_pmc.txt")):
-    """HBM bytes per generation launch from the committed rocprofv3 --pmc
-    summary of this workload (FETCH_SIZE and WRITE_SIZE passes, each scaled
-    by its copy-kernel calibration factor); None when the summary is absent."""
+def measured_traffic(kernel, path=os.path.join(ROOT, "profiles", "mtgp32_items_batched11213_pmc.txt")):
+    """HBM bytes per launch of the generation kernel `kernel` from the
+    committed rocprofv3 --pmc summary of this workload (FETCH_SIZE and
+    WRITE_SIZE passes, each scaled by its copy-kernel calibration factor);
+    None when the summary is absent or of another kernel."""
+    found = {}
     try:
-        for line in open(path):
-            if line.startswith("traffic_bytes_per_launch:"):
-                return int(line.split(":")[1].split()[0])
+        with open(path) as f:
+            for line in f:
+                key, _, value = line.partition(":")
+                if key in ("traffic_kernel", "traffic_bytes_per_launch"):
+                    found[key] = value.split()[0]
     except OSError:
         pass
-    return None
+    if not kernel or found.get("traffic_kernel") != kernel or "traffic_bytes_per_launch" not in found:
+        return None
+    return int(found["traffic_bytes_per_launch"])
 
 
 def main():
@@ -713,7 +719,7 @@ def main():
     # the plan's generation launches (one per word size and state class;
     # this workload has one)
     kernel = max(r["kernels"], key=lambda k: k["items"])["kernel"] if r["kernels"] else None
-    traffic = measured_traffic()
+    traffic = measured_traffic(kernel)
     line = {
         "metric": METRIC,
         "value": round(gbs, 2),
@@ -731,7 +737,7 @@ def main():
         "numbers_per_s": round(r["numbers"] * args.steps / (r["total_ms"] * 1e-3), 1),
         "pct_hbm_peak": round(100 * gbs / HBM_PEAK_GBS, 2),
         "config": {"workload": "batched MTGP32-11213: 128 parameter sets, uneven lengths 2^20..2^26 "
-                               "uint32 + close_open float32 each; per step one jump launch (cell start states) + "
+                               "uint32 + close_open float32 each; per step the jump launches (cell start states) + "
                                "one persistent generation launch",
                    "generators": r["G"], "output_bytes": r["out_bytes"], "numbers": r["numbers"],
                    "work_items": r["stats"]["items"], "launches_per_step": r["stats"]["launches"],
