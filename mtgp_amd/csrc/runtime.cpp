@@ -270,6 +270,26 @@ int Context::per_cu(int bits, int cls, int layout, int cells, int knob) const {
     return b;
 }
 
+int Context::launch_layout(int bits, int cls, int mask, int cells, uint64_t cell, uint64_t numbers, bool one_round,
+                           bool cached, bool &fits) const {
+    const int b = bits == 64, knob = bpc[b][cls];
+    const int model = layout_one_round_for(bits, cls, mask, cells, cell, numbers);
+    // Cells on a cache's grid (a server's batches, often a few dozen cells)
+    // take the model's layout where they are one round of it: bursts of 128
+    // requests 1056 and 1251 us against 1198 and 1370.
+    fits = one_round || (cached && cells <= cus * std::min(knob, blocks_per_cu[b][cls][model]));
+    if (fits)
+        return model;
+    const int lay = layout_for(bits, cls, mask);
+    // Cells that layout 1 holds in one round and that are too short to hide
+    // the claims stay there (4096 MTGP32-11213 cells of 2^12, 2^14, 2^16
+    // words: 21, 54, 233 us against 55, 76, 220).
+    if (layout[b][cls] < 0 && cells <= cus * per_cu(bits, cls, 1, cells, knob) &&
+        gen_ns(*this, bits, cls, 1, cells, cell, numbers) < gen_ns(*this, bits, cls, lay, cells, cell, numbers))
+        return 1;
+    return lay;
+}
+
 int Context::launch_per_cu(int bits, int cls, int layout, int cells, bool one_round) const {
     if (one_round)
         return per_cu(bits, cls, layout, cells, bpc[bits == 64][cls]);
@@ -1761,25 +1781,9 @@ void Plan::build(Context &c, const std::vector<GenRef> &gens, const std::vector<
                     L.numbers += cost[(size_t)order[q]];
                     longest = std::max<uint64_t>(longest, cost[(size_t)order[q]]);
                 }
-                const int knob = c.bpc[L.bits == 64][L.cls];
-                const int model = c.layout_one_round_for(L.bits, L.cls, L.layouts_ok, L.count, longest, L.numbers);
-                // Cells on a cache's grid (a server's batches, often a few
-                // dozen cells) take the model's layout where they are one
-                // round of it: bursts of 128 requests 1056 and 1251 us
-                // against 1198 and 1370.
-                const bool fits =
-                    one_round ||
-                    (opt.cache && L.count <= c.cus * std::min(knob, c.blocks_per_cu[L.bits == 64][L.cls][model]));
-                L.layout = fits ? model : c.layout_for(L.bits, L.cls, L.layouts_ok);
-                // Cells that layout 1 holds in one round and that are too
-                // short to hide the claims stay there (4096 MTGP32-11213
-                // cells of 2^12, 2^14, 2^16 words: 21, 54, 233 us against 55,
-                // 76, 220).
-                if (!fits && c.layout[L.bits == 64][L.cls] < 0 &&
-                    L.count <= c.cus * c.per_cu(L.bits, L.cls, 1, L.count, knob) &&
-                    gen_ns(c, L.bits, L.cls, 1, L.count, longest, L.numbers) <
-                        gen_ns(c, L.bits, L.cls, L.layout, L.count, longest, L.numbers))
-                    L.layout = 1;
+                bool fits;
+                L.layout = c.launch_layout(L.bits, L.cls, L.layouts_ok, L.count, longest, L.numbers, one_round,
+                                           opt.cache != nullptr, fits);
                 const int bpc = c.launch_per_cu(L.bits, L.cls, L.layout, L.count, fits);
                 L.grid = std::min(L.count, c.cus * bpc);
                 L.dyn_lds = c.lds_reserve(kernel_fn(L.bits, L.cls, L.layout), kernel_threads(L.bits, L.cls, L.layout), bpc);

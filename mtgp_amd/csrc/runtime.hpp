@@ -60,6 +60,11 @@ struct Context {
     }
     // The autotuner's for each layout, as it measured them; 0 = not tuned.
     int rounds_tuned[2][4][4] = {};
+    // The layout of a generation launch of `cells` cells, the longest of `cell`
+    // numbers; fits: it runs as one round (one_round: a grid of the model's;
+    // cached: one of a jump cache's).
+    int launch_layout(int bits, int cls, int mask, int cells, uint64_t cell, uint64_t numbers, bool one_round,
+                      bool cached, bool &fits) const;
     // Workgroups per CU of a generation launch, on a one-round grid or any
     // other.
     int launch_per_cu(int bits, int cls, int layout, int cells, bool one_round) const;

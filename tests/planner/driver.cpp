@@ -63,6 +63,16 @@ int planner_tuned(int bits, int cls, int tuned_layout, int tuned, int one_round,
     return c->launch_per_cu(bits, cls, *layout, cells, one_round != 0);
 }
 
+// The layout of a launch of equal cells, of one the model made (1) or a jump
+// cache's grid (2) or any other (0); *fits as launch_layout has it.
+int planner_layout(int bits, int cls, int mask, int cells, uint64_t cell, int grid, int *fits) {
+    std::unique_ptr<Context> c(make());
+    bool f;
+    const int lay = c->launch_layout(bits, cls, mask, cells, cell, (uint64_t)cells * cell, grid == 1, grid == 2, f);
+    *fits = f;
+    return lay;
+}
+
 // Offsets and sizes of a jump's workspace.
 void planner_jump_space(const uint64_t *bytes, uint64_t *out) {
     const JumpSpace W(bytes[0], bytes[1], bytes[2], bytes[3]);

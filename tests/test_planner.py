@@ -28,6 +28,7 @@ def lib():
     lib.planner_sizes.argtypes = one + [C.POINTER(U64), C.c_int]
     lib.planner_ns.argtypes, lib.planner_ns.restype = one + [U64], C.c_double
     lib.planner_cell.argtypes, lib.planner_cell.restype = one, U64
+    lib.planner_layout.argtypes = [C.c_int] * 4 + [U64, C.c_int, C.POINTER(C.c_int)]
     return lib
 
 
@@ -133,3 +134,42 @@ def test_the_host_stages_no_partial_windows(lib, lists, coef, window, parts):
     assert all(o % 256 == 0 for o in (o_coef, o_in, o_out, o_parts))
     assert lists <= o_coef and o_coef + coef <= o_in and o_in + window <= o_out and o_out + window <= o_parts
     assert device == o_parts + parts and host <= lists + coef + 2 * window + 4 * 256
+
+
+def _layout(lib, key, cells, cell, grid=0, mask=None):
+    fits = C.c_int()
+    mask = (3 if key == (64, 3) else 15) if mask is None else mask
+    return lib.planner_layout(*key, mask, cells, cell, grid, C.byref(fits)), fits.value
+
+
+@pytest.mark.parametrize("key", CLASSES)
+def test_launches_of_several_rounds(lib, key):
+    """Long cells take the widest layout that the sets admit; cells that layout
+    1 holds in one round (12 per CU, 8 in the narrow class, and up to half as
+    many again) and that are short stay in layout 1."""
+    top = 1 if key == (64, 3) else 3
+    one = 256 * min(8 if key == (64, 3) else 12, LIMITS[key][1])
+    edge = min(3 * one // 2, 256 * LIMITS[key][1])
+    assert _layout(lib, key, 100 * one, 1 << 17) == (top, 0)
+    assert _layout(lib, key, edge, 4096) == (1, 0)
+    assert _layout(lib, key, edge + 1, 4096) == (top, 0)
+    assert _layout(lib, key, edge, 1 << 22) == (top, 0)
+    for mask, lay in ((3, 1), (7, min(top, 2))):
+        assert _layout(lib, key, 100 * one, 1 << 17, mask=mask & (3 if top == 1 else 15))[0] == lay
+
+
+def test_short_cells_in_one_round_of_layout_1(lib):
+    """The measured line: 4096 MTGP32-11213 cells of 2^12, 2^14, 2^17."""
+    assert [_layout(lib, (32, 0), 4096, 1 << k)[0] for k in (12, 14, 17)] == [1, 1, 3]
+
+
+@pytest.mark.parametrize("key", CLASSES)
+def test_grids_of_one_round(lib, key):
+    """A jump cache's grid runs as the model's while it is one round of it."""
+    for cells in (1, 64, 256, 512):
+        model = _layout(lib, key, cells, 1 << 17, 1)
+        assert model[1] == 1 and _layout(lib, key, cells, 1 << 17, 2) == model
+        if key != (64, 3):
+            assert model[0] == 3 or cells > 256  # few cells: the shortest chain
+    assert _layout(lib, key, 256 * 16 * 12, 1 << 17, 2)[1] == 0
+    assert _layout(lib, key, 256 * 16 * 12, 1 << 17, 1)[1] == 1
