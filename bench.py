@@ -396,7 +396,7 @@ def run_configs(M):
     d = line(S * 4 * count, jump_ms, gen_ms, plan.stats()["items"], substream_setup_ms=round(setup_ms, 3),
              substream_setup_first_ms=round(first_ms, 3),
              workload="4096 substreams i*3^162 of MTGP32-11213 set 0 (seed 777), 2^20 uint32 each, end to end: "
-                      "substream start states made on the device as one matrix-core group (the 4095 states "
+                      "substream start states made on the device, every one a jump from the base (the 4095 states "
                       "J^(i 3^162) w0 as fp4 products of coefficient blocks with the base window's bit planes, and their folds; "
                       "host time included, wall clock, median of 3 calls after the first, which also builds the "
                       "coefficient rows: substream_setup_first_ms) + generation")

@@ -103,8 +103,8 @@ struct Transpose {
 // generated in LDS (kJbBlock numbers past the window), one 32-bit plane of it
 // transposed to bit planes and expanded to fp4 operands (A: bit p of 32
 // consecutive positions is 16 bytes), the tile's coefficients expanded to B.
-// Then each wave takes word groups: 8 accumulators for 8 consecutive window
-// words.  The operand of word j is the bit planes from position j on: dword
+// Then each wave takes word groups: kTileWords consecutive window words, an
+// accumulator each per column tile (4 or 8).  The operand of word j is the bit planes from position j on: dword
 // r of it holds the bits at offsets 4 q + r, so word j + 1's is the same
 // four dwords moved on by one with one new dword (a funnel shift of the
 // expanded planes).
@@ -377,7 +377,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void jump_tiles_kernel(const JumpB
 
 // ------------------------------------------------------------------- folds
 // One workgroup per JumpFold: T threads, S numbers per step.  The chain of a
-// block is 1 to 4 steps, no longer than a load of its part can take (the
+// block is 1 to 4 steps (8 in the narrow class), about as long as a load of its part can take (the
 // tiles wrote it from any XCD, so it misses the L2), so parts are loaded
 // kFoldAhead blocks ahead (one and four ahead, one jump: MTGP32-11213 8.8 and
 // 7.6 us, MTGP64-23209 19.8 and 16.9, MTGP64-44497 28.5 and 24.4, MTGP64-

@@ -159,7 +159,7 @@ void jump_noalloc(mtgp32_fast_t *g, const char *hex) {
     hip_check(hipMemcpy(base + kItemOff, ji, (size_t)(parts + 1) * sizeof(JumpItem), hipMemcpyHostToDevice),
               "hipMemcpy items");
     hip_check(hipMemcpy(base + kParamOff, &rec, sizeof(rec), hipMemcpyHostToDevice), "hipMemcpy param");
-    // The kernels' work-queue pairs must be zero on entry (a launch leaves
+    // The kernels' work-queue counters must be zero on entry (a launch leaves
     // its pair zero, but one that failed part-way may not have).
     hip_check(hipMemsetAsync(base + kQueueOff, 0, 4 * sizeof(uint32_t), 0), "hipMemsetAsync queue");
     const JumpItem *items = reinterpret_cast<const JumpItem *>(base + kItemOff);

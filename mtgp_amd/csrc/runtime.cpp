@@ -1914,7 +1914,8 @@ void Plan::launch_part(int part, hipStream_t s) { run_launches(part, -1, s); }
 
 void Plan::launch_phase(int part, int phase, hipStream_t s) { run_launches(part, phase, s); }
 
-// Work-queue counter pairs: [launches | jlaunches | mlaunches | mjlaunches].
+// Work-queue counters, one per launch, 8 bytes apart: [launches | jlaunches |
+// mlaunches | mjlaunches].
 void Plan::run_launches(int part, int phase, hipStream_t s) {
     const bool merged = phase < 0;
     const auto &J = merged ? mjlaunches : jlaunches;
@@ -2253,7 +2254,7 @@ static void device_jump(Context &c, int slot, int bits, int mexp, const void *in
     cj.state_bytes = wbytes;
     if (host_io)
         memcpy(h + o_in, in, (size_t)wbytes);
-    // the queue pairs go up as zeros with the rest
+    // the queue counters go up as zeros with the rest
     hip_check(hipMemcpyAsync(d, h, up, hipMemcpyHostToDevice, nullptr), "hipMemcpyAsync jump workspace");
     const int cls = c.class_of(slot);
     const JumpItem *d_items = reinterpret_cast<const JumpItem *>(d + o_items);
@@ -3060,7 +3061,13 @@ int mtgp_genset_jump(mtgp_genset_t *s, int g, const char *hex) {
 // (substream 0's slot 0) jumped by J^t.
 //  - MTGP32 sets of more than kDirectSubstreams: every substream one jump from
 //    the base, J^t for t < G made on the host pool once per jump string, as
-//    the reference keeps its 4^k 3^162 table.
+//    the reference keeps its 4^k 3^162 table.  Such a call is the faster one
+//    for any number of substreams (MTGP32-11213, 65, 257 and 1500: 32, 41, 105
+//    us against 78, 106, 246 by levels; MTGP64-23209 54, 87, 324 against 129,
+//    206, 560), but the first one with a string waits for its polynomials
+//    (MTGP32-11213 2.1, 4.4, 5 to 9 ms against 0.5, 0.7, 1.2 to 2; MTGP64-23209
+//    6.5, 13, 24 against 1.5, 2.1, 2.7), so small sets, and the dearer MTGP64
+//    ones, which gain less for it, take the levels.
 //  - others: radix-4 levels, level m making t = a 4^m + j (a = 1..3, j < 4^m)
 //    as J^(a 4^m) applied to substream j -- the decomposition of t in powers of
 //    J the reference's substream samples use (openCL-sample/mtgp32-jump.cl:

@@ -50,7 +50,11 @@ struct Context {
     // occupancy limit): the knob (bpc) halved or quartered, but whole where
     // layout 3 then has two rounds at most (6 and 8 per CU: 3072 and 4096
     // MTGP32-11213 cells of 17 GB 3576, 3384 and 3352, 3314 us; 6000, 8192
-    // 3155, 3126 and 3246, 3158; 4096 of MTGP32-23209 3226 and 3139).
+    // 3155, 3126 and 3246, 3158; 4096 of MTGP32-23209 3226 and 3139).  In
+    // layout 3 the half: 64 streams in 16384 to 32768 cells whole / half /
+    // quarter, MTGP32-11213 4761 / 4783 / 5746 us, MTGP32-23209 9431 / 9438 /
+    // 9728, MTGP64-23209 6531 / 6503 / 6888; MTGP64-44497 a quarter, 13910 /
+    // 13937 / 13835; in the largest classes they are even.
     int rounds_knob(int bits, int cls, int layout, int cells) const {
         if (rounds_tuned[bits == 64][cls][layout] > 0)
             return rounds_tuned[bits == 64][cls][layout];
@@ -76,7 +80,11 @@ struct Context {
     // The layout whose occupancy and waves size the cells of such grids: more
     // cells would cost more jumps than the even finish gains (the two-size
     // grid of the batched MTGP32-11213 workload for 6, 8 and 12 cells per CU
-    // in a round: 3.86, 3.83, 3.77 ms).
+    // in a round: 3.86, 3.83, 3.77 ms).  64 streams of 16 GiB, sized as for
+    // layouts 1 / 2 / 3: MTGP32-11213 3.53 / 3.68 / 5.80 ms, MTGP32-23209 4.53
+    // / 4.26 / 5.00, MTGP64-23209 4.57 / 4.27 / 5.43.  The larger states take
+    // the two-size grid only where it is forced or the job is longer than any
+    // measured (one round there: MTGP32-44497 3.98 against 5.6 to 6.0).
     static constexpr int sizing[2][4] = {{1, 2, 3, 1}, {2, 3, 2, 1}};
     // The same for one-round grids; -1 = the layout that the step-time model
     // (gen_ns) has fastest for the launch's cells.  Few cells leave each CU a
@@ -508,17 +516,7 @@ struct Plan {
     // of multi-wave layouts divided by their waves.
     bool waves_scaled = false;
     bool one_round_grid = false;  // cells from the step-time model, one round
-    bool overlap = false;
-    // Batched jumps are split into partial jumps (chunk ranges, XORed when
-    // the generation kernel loads the start window) until a jump launch has
-    // about this many waves per CU: a jump launch is one round of waves, so
-    // its duration is one wave's share of the chunks.
-    int jump_waves_per_cu = 16;
-    // Most partial jumps one batched jump is split into (each reads and
-    // XORs its partial window when the generation kernel loads the cell).
-    // 16 measured best: one MTGP32-11213 stream (1017 jumps) 0.195 ms per
-    // jump launch against 0.25 ms at 8; batches unchanged.
-    int jump_max_parts = 16;     // launch() uses the two-phase order
+    bool overlap = false;         // launch() uses the two-phase order
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
 

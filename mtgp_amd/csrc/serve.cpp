@@ -229,8 +229,9 @@ struct mtgp_server {
         o.stream = streams[(size_t)B.stream];
         o.sync = false;
         o.jump_mode = (cfg.flags & MTGP_SERVER_FUSED_JUMPS) ? 0 : 1;
-        // Batches carry few jumps: split each down to one chunk per wave so
-        // a jump takes about one chunk's fold instead of several.
+        // Word-XOR jumps (jump_mfma_min above a batch's few): each is split
+        // down to one chunk per wave, so that it takes about one chunk's fold
+        // instead of several.
         o.max_parts = 64;
         const auto tp = Clock::now();
         B.plan.build(*ctx, B.refs, B.rq, o);
