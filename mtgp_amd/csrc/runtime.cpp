@@ -1018,7 +1018,7 @@ uint64_t table_cell(uint64_t longest, int gens, uint64_t S) {
     };
     if (!worth(S))
         return 0;
-    const uint64_t T = octave_size(S, gens == 1 ? 4 : 8);
+    const uint64_t T = octave_size(S, gens == 1 ? 4 : 16);
     return worth(T) ? T : 0;
 }
 

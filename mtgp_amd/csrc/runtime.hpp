@@ -297,10 +297,13 @@ inline uint64_t octave_size(uint64_t v, uint64_t steps) {
 // call of another length found no table and made one on the host (calls 0 to
 // 2% shorter than n, exact sizes and these: one MTGP32-23209 stream of 10^6
 // numbers 3.04 and 0.10 ms a call, two of 5 * 10^5 2.4 and 0.10 ms; one
-// MTGP64-110503 stream of 2^24 38 and 0.47 ms).  4 sizes an octave cost one
-// stream 0.7% of its modelled step time at most, on average over a decade of
-// lengths, 8 cost a few streams 1.5%; more streams or longer cells, whose
-// repeated calls would lose up to 7%, keep the exact sizes.
+// MTGP64-110503 stream of 2^24 38 and 0.47 ms).  Repeated calls of
+// one stream take 0.999 of the exact sizes' time with 4 sizes an octave (mean
+// of 16 lengths in each of 8 sets, 1.041 at worst; 8: 0.995, 1.039), of four
+// streams 0.998 with 16 (1.021; 8: 1.002, 1.073); more sizes find a table less
+// often (60 lengths over a decade from 10^5, one MTGP64-44497 stream: exact 4.2
+// ms a call, 16, 8, 4 sizes 2.2, 1.9, 1.1).  More streams, or longer cells, keep exact
+// sizes.
 uint64_t table_cell(uint64_t longest, int gens, uint64_t S);
 // The cell sizes that a one-round grid is chosen from, each once, largest
 // first: the longest stream in 1, 2, 3, ... parts (one part = no jumps at

@@ -94,13 +94,13 @@ def test_streams_of_many_cells_take_table_sizes(lib, key):
 @pytest.mark.parametrize("gens,parts", [(2, 4), (16, 4), (17, 16), (64, 16)])
 def test_sets_take_table_sizes_for_many_short_cells(lib, gens, parts):
     """From `parts` cells each on, of 2^17 numbers at most; the rounding may
-    cost one cell in 9."""
+    cost one cell in 17."""
     n = 1 << 22 if gens < 17 else 1 << 20
     sizes = _sizes(lib, (64, 0), [n + 1] * gens)
-    assert all(_is_table_size(s, 8) for s in sizes if n // s >= parts + parts // 4 and s <= 7 << 14)
-    assert any(not _is_table_size(s, 8) for s in sizes if 1 < n // s < parts), sizes
+    assert all(_is_table_size(s, 16) for s in sizes if n // s >= parts + parts // 4 and s <= 7 << 14)
+    assert any(not _is_table_size(s, 16) for s in sizes if 1 < n // s < parts), sizes
     sizes = _sizes(lib, (64, 0), [1 << 25] * 64)
-    assert any(s > 1 << 17 and not _is_table_size(s, 8) for s in sizes)
+    assert any(s > 1 << 17 and not _is_table_size(s, 16) for s in sizes)
 
 
 @pytest.mark.parametrize("key", CLASSES)
