@@ -36,6 +36,9 @@ def test_plans(mtgp, oracle, spec, cells):
     with mtgp.tuning(jump_mfma_min=0):
         plan = gs.plan([(g, 0, count, 0, b) for g, b in enumerate(bufs)], segment=4096)
     assert plan.stats()["jumps"] == 2 * (cells - 1) and plan.stats()["matrix_jumps"] == 0
+    # one jump launch and one of generation; blocked jumps have two
+    assert plan.stats()["launches"] == 2
+    assert gs.plan([(g, 0, count, 0, b) for g, b in enumerate(bufs)], segment=4096).stats()["launches"] == 3
     want = [oracle.generate(p, oracle.init_state(p, 50 + g), 0, count) for g in range(2)]
     for _ in range(2):
         for b, (e, _w) in zip(bufs, want):
